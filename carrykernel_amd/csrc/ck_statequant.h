@@ -9,6 +9,7 @@
 #include "ck_capi_common.h"
 #include "ck_device.h"
 #include "ck_quant.h"
+#include "ck_tiles.h"
 
 namespace ck {
 namespace qs {
@@ -17,8 +18,6 @@ constexpr int kResFp32 = CK_RES_FP32;
 constexpr int kResFp16 = CK_RES_FP16;
 constexpr int kResFp8 = CK_RES_FP8;
 constexpr int kResInt8 = CK_RES_INT8;
-
-constexpr int kGroups = 32;  // column groups per workgroup (one half-wave)
 
 // K-slices per workgroup, one half-wave each.
 template <int K>
@@ -139,23 +138,6 @@ __device__ __forceinline__ void st_b16(uint16_t* p, const uint32_t (&w)[(CPT + 1
   else *p = (uint16_t)w[0];
 }
 
-// How a workgroup's threads are laid over a tile's columns and the K-slices.
-//  kTileFull: 32 groups of 4 columns.
-//  kTileAny: G <= 40 (K = 256, whose 16 slices would take 640 threads and spill:
-//    32) groups of 4 columns, G and the number of threads (S * G
-//    rounded up to whole waves) set per launch, so a head of any V >= 4 wastes
-//    only the last wave's rest.
-//  kTileOne: 32 single columns, for V < 4 and V > 2^21.
-// The tiles of a matrix are of equal width (a multiple of 4), so the last one
-// never has fewer than 4 columns and its last thread can take the 4 that end
-// with V, sharing some with its neighbour; the threads past S * G repeat the
-// last one's work. What is computed twice has the same value from the same
-// inputs, and every input of a workgroup is read before it stores (a barrier
-// lies between), which in-place use needs.
-enum TileForm : int { kTileFull, kTileAny, kTileOne };
-
-constexpr int max_groups(int KP) { return KP <= 128 ? 40 : 32; }
-
 template <int FORM, int KP>
 struct TileShape {
   static constexpr int CPT = FORM == kTileOne ? 1 : 4;
@@ -167,32 +149,6 @@ struct TileShape {
 // that it is one register beside a uniform base per row, and 64 in the form that heads too wide for it take.
 template <int FORM>
 using LaneOffset = std::conditional_t<FORM == kTileOne, int64_t, uint32_t>;
-constexpr int kMaxTileV = 1 << 21;
-
-struct ColTiles {
-  int nvt, width;   // tiles and columns per tile (the last one: what is left)
-  int groups;       // column groups per tile
-  uint32_t inv;     // ceil(2^16 / groups): t / groups = t * inv >> 16 for t < 1024
-  TileForm form;
-};
-
-// fp32_rows: the rows' largest elements are fp32; a tile of 24 groups or more is
-// then better left in the full form (HV=32, K=128, V=96, B=40, us, full / any: fp32
-// step 20.3 / 22.3, fp32 residual 31.8 / 32.8; fp16 21.4 / 20.3, fp8 17.3 / 15.9).
-inline ColTiles col_tiles(int V, int KP, bool fp32_rows) {
-  const int cpt = V >= 4 && V <= kMaxTileV ? 4 : 1;
-  const int all = (V + cpt - 1) / cpt;  // column groups
-  const int rest = V % (kGroups * 4);
-  const bool full = rest == 0 || (fp32_rows && V % 4 == 0 && rest >= 96);
-  const int most = cpt == 4 && !full ? max_groups(KP) : kGroups;
-  const int nvt = (all + most - 1) / most;
-  const int groups = cpt == 4 && !full ? (all + nvt - 1) / nvt : kGroups;
-  return ColTiles{nvt, groups * cpt, groups, (65536u + groups - 1) / groups,
-                  cpt == 1 ? kTileOne : full ? kTileFull : kTileAny};
-}
-
-// Threads of a workgroup with S slices.
-inline int tile_threads(const ColTiles& t, int S) { return (t.groups * S + 63) / 64 * 64; }
 
 // A thread's place in its tile: column group, slice, first column (-1: none).
 struct TilePlace {
@@ -221,15 +177,6 @@ __device__ __forceinline__ uint32_t pack_codes(const uint32_t (&yb)[CPT]) {
   if constexpr (CPT == 4) return pack_low_bytes(yb[0], yb[1], yb[2], yb[3]);
   else return yb[0] & 0xffu;
 }
-
-// K padded to KP = max(16, next_pow2(K)) (K <= 256)
-inline int padded_k(int K) {
-  int kp = 16;
-  while (kp < K) kp *= 2;
-  return kp;
-}
-
-inline bool valid_k(int K) { return K >= 1 && K <= 256; }
 
 // Bitwise OR of the addresses: its low bits are zero only if every pointer is
 // aligned that far.

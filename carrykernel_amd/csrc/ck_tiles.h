@@ -1,0 +1,75 @@
+// How the kernels of the statequant layout split a matrix's V columns over
+// workgroups. Host rules only, plain C++: tests/test_column_tiles_cpu.py compiles
+// this header by itself.
+#pragma once
+
+#include <stdint.h>
+
+namespace ck {
+namespace qs {
+
+constexpr int kGroups = 32;  // column groups per workgroup (one half-wave)
+
+// How a workgroup's threads are laid over a tile's columns and the K-slices.
+//  kTileFull: 32 groups of 4 columns.
+//  kTileAny: G <= 40 (K = 256, whose 16 slices would take 640 threads and spill:
+//    32) groups of 4 columns, G and the number of threads (S * G
+//    rounded up to whole waves) set per launch, so a head of any V >= 4 wastes
+//    only the last wave's rest.
+//  kTileOne: 32 single columns, for V < 4 and V > 2^21.
+// The tiles of a matrix are of equal width (a multiple of 4) and the last one has
+// at least 4 columns, so its last thread can take the 4 that end with V, sharing
+// some with its neighbour in the same workgroup; the threads past S * G repeat the
+// last one's work. What is computed twice has the same value from the same
+// inputs, and every input of a workgroup is read before it stores (a barrier
+// lies between), which in-place use needs. Columns shared by two workgroups would
+// break that: one could read what the other has stored.
+enum TileForm : int { kTileFull, kTileAny, kTileOne };
+
+constexpr int max_groups(int KP) { return KP <= 128 ? 40 : 32; }
+
+constexpr int kMaxTileV = 1 << 21;
+
+struct ColTiles {
+  int nvt, width;   // tiles and columns per tile (the last one: what is left)
+  int groups;       // column groups per tile
+  uint32_t inv;     // ceil(2^16 / groups): t / groups = t * inv >> 16 for t < 1024
+  TileForm form;
+};
+
+// fp32_rows: the rows' largest elements are fp32; a tile of 24 groups or more is
+// then better left in the full form (HV=32, K=128, V=96, B=40, us, full / any: fp32
+// step 20.3 / 22.3, fp32 residual 31.8 / 32.8; fp16 21.4 / 20.3, fp8 17.3 / 15.9).
+inline ColTiles col_tiles(int V, int KP, bool fp32_rows) {
+  const int cpt = V >= 4 && V <= kMaxTileV ? 4 : 1;
+  const int all = (V + cpt - 1) / cpt;  // column groups
+  const int rest = V % (kGroups * 4);
+  const bool full = rest == 0 || (fp32_rows && V % 4 == 0 && rest >= 96);
+  const bool any = cpt == 4 && !full;
+  int groups = kGroups;
+  int nvt = (all + groups - 1) / groups;
+  // the fewest tiles, of as many groups as that needs; fewer where that leaves the
+  // last tile one group of fewer than 4 columns (V = 6241: 40 tiles of 40 groups)
+  for (int most = any ? max_groups(KP) : 0; most > 0; --most) {
+    nvt = (all + most - 1) / most;
+    groups = (all + nvt - 1) / nvt;
+    if (V - (nvt - 1) * groups * 4 >= 4) break;
+  }
+  return ColTiles{nvt, groups * cpt, groups, (65536u + groups - 1) / groups,
+                  cpt == 1 ? kTileOne : full ? kTileFull : kTileAny};
+}
+
+// Threads of a workgroup with S slices.
+inline int tile_threads(const ColTiles& t, int S) { return (t.groups * S + 63) / 64 * 64; }
+
+// K padded to KP = max(16, next_pow2(K)) (K <= 256)
+inline int padded_k(int K) {
+  int kp = 16;
+  while (kp < K) kp *= 2;
+  return kp;
+}
+
+inline bool valid_k(int K) { return K >= 1 && K <= 256; }
+
+}  // namespace qs
+}  // namespace ck

@@ -92,3 +92,10 @@ def test_very_wide_head():
     for a, b in zip(got, ref):
         if a is not None:
             np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("K,V", [(128, 6241), (256, 3969)])
+def test_wide_ragged_heads(K, V):
+    """Heads whose columns once left the last tile a single ragged group, in place
+    and out of place."""
+    test_step(K, V)
