@@ -411,7 +411,7 @@ template <int FORM>
 void launch_cols_form(const ColsParams& p, int KP, int64_t M, bool ieee, hipStream_t s) {
   if (KP != p.K) launch_cols<FORM, true, true>(p, KP, M, s);
   else if (ieee) launch_cols<FORM, false, true>(p, KP, M, s);
-  else if constexpr (FORM != qs::kTileOne) launch_cols<FORM, false, false>(p, KP, M, s);  // V % 4 == 0
+  else launch_cols<FORM, false, false>(p, KP, M, s);  // V % 4 == 0: kTileOne for a V past kMaxTileV
 }
 
 // K above 256: one thread per (matrix, V-column); consecutive threads take

@@ -67,3 +67,17 @@ def test_infinities_and_huge_values(K, V):
     assert torch.equal(codes[1, :, 2:3], huge) and torch.equal(scale[1, 2:3], s_huge)
     cols = [c for c in range(V) if c not in (1, 2)]
     assert torch.equal(codes[:, :, cols], ref[:, :, cols])
+
+
+def test_very_wide_matrix():
+    """V past the four-column tiles' limit, a multiple of 4, aligned, K a power
+    of two: one column per thread in the non-IEEE arithmetic."""
+    K, V = 16, (1 << 21) + 4
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(K, V, generator=g, device="cuda") * 0.3
+    codes, scale = _expect(x, 127.0)
+    got = sq.per_v_channel_quantize(x)
+    for name, a, b in zip(("codes", "scale", "deq"), got, (codes, scale, codes.float() * scale[None, :])):
+        assert torch.equal(a, b), name
+    c, s, e, es = sq.init_quant_state(x[None, None], res_fmt=sq.RES_INT8)
+    assert torch.equal(c[0, 0], codes) and torch.equal(s[0, 0], scale) and not e.any() and not es.any()
