@@ -499,9 +499,10 @@ __device__ __forceinline__ void process_item(const PackedParams& p, const ItemCo
   constexpr int RKL = L::RK / LPR;  // residual bytes per lane
   // masked rows: waves past V (a tile's rows rounded up) skip the row work
   const int wave_row = MASKED ? ic.vt * L::ROWS_WG + wave * L::ROWS_WAVE : 0;
-  // byte offsets of the lane's first row, the further ones a uniform step away
-  const uint32_t soff = MASKED ? (uint32_t)(row0 * KA + c * 16) : 0u;
-  const uint32_t eoff = MASKED ? (uint32_t)(row0 * RKA + c * RKL) : 0u;
+  // byte offsets of the lane's first row (unsigned: a row past V may lie past
+  // 2^31), the further ones a uniform step away
+  const uint32_t soff = MASKED ? (uint32_t)row0 * (uint32_t)KA + c * 16u : 0u;
+  const uint32_t eoff = MASKED ? (uint32_t)row0 * (uint32_t)RKA + (uint32_t)(c * RKL) : 0u;
   int8_t* sbase = p.state + dslot * p.stride_state + (int64_t)ic.hv * p.V * KA;
   int8_t* ebase = p.resid + dslot * p.stride_resid + (int64_t)ic.hv * p.V * RKA;
   float* scb = p.sscale + dslot * p.stride_sscale + (int64_t)ic.hv * p.V;

@@ -13,6 +13,7 @@
 // of the power-of-two K of real models, this one every other shape.
 #pragma once
 
+#include "ck_row_offset.h"
 #include "packed_decode_impl.h"
 
 namespace ck {
@@ -114,14 +115,12 @@ __device__ __forceinline__ void load_item_masked(const PackedParams& p, const It
       for (int j = 0; j < L::EW; ++j) R.ew[i][j] = 0u;
     }
     if (c * 16 < K) {
-      // one product per region: the further rows are a uniform step away
-      const int s0 = row0 * K, e0 = row0 * RKA;
       // K >= 16 here, so the piece that ends with the row starts inside it
       const int sc = min(c * 16, K - 16), ec = min(c * RKL, RKA - RKL);
 #pragma unroll
       for (int i = 0; i < RPL; ++i) {
-        R.cw[i] = ld_16_u<STREAM>(sbase + (uint32_t)(min(s0 + i * L::RPI * K, (p.V - 1) * K) + sc));
-        const int8_t* e = ebase + (uint32_t)(min(e0 + i * L::RPI * RKA, (p.V - 1) * RKA) + ec);
+        R.cw[i] = ld_16_u<STREAM>(sbase + (clamped_row_offset(row0, i * L::RPI, K, p.V) + (uint32_t)sc));
+        const int8_t* e = ebase + (clamped_row_offset(row0, i * L::RPI, RKA, p.V) + (uint32_t)ec);
         if constexpr (RESID == kResidInt4) {
           const u32x2 e2 = ld_8_u<STREAM>(e);
           R.ew[i][0] = e2.x, R.ew[i][1] = e2.y;
