@@ -9,6 +9,7 @@
 #include <string>
 
 #include "carrykernel_gdn.h"
+#include "ck_launch.h"
 
 namespace ck {
 

@@ -308,13 +308,14 @@ int launch_fs_cfg(PackedParams p, int B, hipStream_t stream) {
   const int64_t items = (int64_t)B * p.HV * nvt;
   if (items > 0x7fffffff) return fail(CK_EUNSUPPORTED, "%lld work items is too many", (long long)items);
   if (items == 0) return ok();
-  const int64_t cap = pd::max_items_override();
-  if (cap > 0 && items > cap) {  // consecutive launches over slices of the requests
+  const int64_t cap = pd::one_item_cap(WAVES * 64);
+  if (items > cap) {  // consecutive launches over slices of the requests
     const int64_t per_request = (int64_t)p.HV * nvt;
     if (per_request > cap) return fail(CK_EUNSUPPORTED, "%lld work items per request is too many", (long long)per_request);
     const int chunk = (int)(cap / per_request);
-    for (int n0 = 0; n0 < B; n0 += chunk) {
-      const int rc = launch_fs_cfg<K, RPL, BF16, ACT>(pd::requests_from(p, n0), min(chunk, B - n0), stream);
+    for (int64_t n0 = 0; n0 < B; n0 += chunk) {
+      const int n = (int)min((int64_t)chunk, B - n0);
+      const int rc = launch_fs_cfg<K, RPL, BF16, ACT>(pd::requests_from(p, (int)n0), n, stream);
       if (rc != CK_OK) return rc;
     }
     return ok();
@@ -330,13 +331,13 @@ int launch_fs_cfg(PackedParams p, int B, hipStream_t stream) {
 
 // Two rows per lane from 512 such tiles on, below that one (a small batch over
 // more SIMDs), as the quantized decode with per-row scales; also two where a
-// request's smaller tiles would pass the process's limit of items per launch.
+// request's smaller tiles would pass the limit of items per launch.
 template <int K, bool BF16, int ACT>
 int launch_fs(const PackedParams& p, int B, hipStream_t stream) {
   constexpr int TILE = FLayout<K, 2, 4>::ROWS_WG;
-  const int64_t cap = pd::max_items_override();
+  const int64_t cap = pd::one_item_cap(4 * 64);
   const int64_t small = (int64_t)p.HV * ((2 * (int64_t)p.V + TILE - 1) / TILE);
-  if ((int64_t)B * p.HV * ((p.V + TILE - 1) / TILE) >= 512 || (cap > 0 && small > cap))
+  if ((int64_t)B * p.HV * ((p.V + TILE - 1) / TILE) >= 512 || small > cap)
     return launch_fs_cfg<K, 2, BF16, ACT>(p, B, stream);
   return launch_fs_cfg<K, 1, BF16, ACT>(p, B, stream);
 }

@@ -514,15 +514,19 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   const uintptr_t bits = qs::addr_bits(x, codes, scale);
   const int KP = K <= 256 ? qs::padded_k(K) : 0;
   const qs::ColTiles tiles = qs::col_tiles(V, KP, true);
-  if (K <= 256 && M <= 0x7fffffff / tiles.nvt) {
-    const ColsParams p{x, V, tiles, K, qmax, codes, scale, deq, static_cast<char*>(e), e_bytes, e_scale};
+  if (K <= 256) {
     const bool ieee = qs::ingest_ieee(bits, M, K, V);
-    switch (tiles.form) {
-      case qs::kTileFull: launch_cols_form<qs::kTileFull>(p, KP, M, ieee, s); break;
-      case qs::kTileAny: launch_cols_form<qs::kTileAny>(p, KP, M, ieee, s); break;
-      default: launch_cols_form<qs::kTileOne>(p, KP, M, ieee, s); break;
-    }
-    return check_launch("ck_quantize_cols");
+    return launch_slices(M, tiles.nvt, qs::tile_threads(tiles, KP <= 128 ? 8 : 16), [&](int64_t m0, int64_t n) {
+      const int64_t i = m0 * K * V, c = m0 * V;  // the slice's first matrix and column
+      const ColsParams p{x + i, V, tiles, K, qmax, codes + i, scale + c, deq ? deq + i : nullptr,
+                         e ? static_cast<char*>(e) + i * e_bytes : nullptr, e_bytes, e_scale ? e_scale + c : nullptr};
+      switch (tiles.form) {
+        case qs::kTileFull: launch_cols_form<qs::kTileFull>(p, KP, n, ieee, s); break;
+        case qs::kTileAny: launch_cols_form<qs::kTileAny>(p, KP, n, ieee, s); break;
+        default: launch_cols_form<qs::kTileOne>(p, KP, n, ieee, s); break;
+      }
+      return check_launch("ck_quantize_cols");
+    });
   }
   const int64_t grid = (M * V + 255) / 256;
   if (grid > 0x7fffffff) return fail(CK_EUNSUPPORTED, "too many columns");

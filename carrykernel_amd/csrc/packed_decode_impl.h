@@ -1011,6 +1011,12 @@ inline int64_t launch_item_cap(int resident, int per_cu) {
   return cap;
 }
 
+// Items that a launch of one workgroup of `threads` threads per item may hold.
+inline int64_t one_item_cap(int threads) {
+  const int64_t cap = max_workgroups(threads), v = max_items_override();
+  return v > 0 && v < cap ? v : cap;
+}
+
 // The same step for requests n0 .. of p: per-request inputs, outputs and ids
 // advanced by n0 requests (the pool and the per-head inputs are shared).
 inline PackedParams requests_from(const PackedParams& p, int n0) {
@@ -1224,16 +1230,16 @@ int launch_cfg(PackedParams p, int B, hipStream_t stream) {
   const int forced = decode_kernel_override();
   if (forced != kDecodeKernelAuto) single = forced == kDecodeKernelOneItem;
   // the persistent kernel's gate table bounds its items per launch; the
-  // one-item kernel has no table, so only a process-wide limit splits it
-  const int64_t override_cap = max_items_override();
-  const int64_t cap = single ? (override_cap > 0 ? override_cap : items) : launch_item_cap(resident, per_cu);
+  // one-item kernel has no table, so only a launch's work items and a
+  // process-wide limit split it
+  const int64_t cap = single ? one_item_cap(WAVES * 64) : launch_item_cap(resident, per_cu);
   if (items > cap) {  // consecutive launches over slices of the requests
     const int64_t per_request = (int64_t)p.HV * nvt;
     if (per_request > cap) return fail(CK_EUNSUPPORTED, "%lld work items per request is too many", (long long)per_request);
     const int chunk = (int)(cap / per_request);
-    for (int n0 = 0; n0 < B; n0 += chunk) {
-      const int rc = launch_cfg<K, RPL, WAVES, RESID, PER_HEAD, MODE, ACT, DST>(requests_from(p, n0), min(chunk, B - n0),
-                                                                              stream);
+    for (int64_t n0 = 0; n0 < B; n0 += chunk) {
+      const int n = (int)min((int64_t)chunk, B - n0);
+      const int rc = launch_cfg<K, RPL, WAVES, RESID, PER_HEAD, MODE, ACT, DST>(requests_from(p, (int)n0), n, stream);
       if (rc != CK_OK) return rc;
     }
     return ok();

@@ -183,6 +183,18 @@ int launch_masked_cfg(PackedParams p, int B, hipStream_t stream) {
   const int64_t items = (int64_t)B * p.HV * nvt;
   if (items > 0x7fffffff) return fail(CK_EUNSUPPORTED, "%lld work items is too many", (long long)items);
   if (items == 0) return ok();
+  const int64_t per_request = (int64_t)p.HV * nvt, most = max_workgroups(WAVES * 64);
+  if (items > most) {  // consecutive launches over slices of the requests
+    if (per_request > most) return fail(CK_EUNSUPPORTED, "%lld work items per request is too many", (long long)per_request);
+    const int chunk = (int)(most / per_request);
+    for (int64_t n0 = 0; n0 < B; n0 += chunk) {
+      const int n = (int)min((int64_t)chunk, B - n0);
+      const int rc = launch_masked_cfg<KP, RPL, WAVES, RESID, PER_HEAD, MODE, DST, MASK>(requests_from(p, (int)n0), n,
+                                                                                       stream);
+      if (rc != CK_OK) return rc;
+    }
+    return ok();
+  }
   p.items = (int)items;
   p.div_nvt = make_fastdiv((uint32_t)nvt);
   p.div_hv = make_fastdiv((uint32_t)p.HV);

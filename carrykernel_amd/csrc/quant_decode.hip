@@ -311,11 +311,16 @@ extern "C" int ck_gdn_quant_decode(const float* h0, int8_t* h, float* scale, voi
   const int64_t heads = (int64_t)B * HV;
   const int cols = kDecodeWaves * (K <= 128 ? 8 : 4);  // columns per workgroup
   const int nvt = (V + cols - 1) / cols;
-  if (heads * nvt > 0x7fffffff) return fail(CK_EUNSUPPORTED, "grid too large");
+  if (heads > 0x7fffffff) return fail(CK_EUNSUPPORTED, "too many heads");
   volatile float one = 1.0f;
-  const DecodeParams p{h0, h, scale, e, e_scale, q, k, v, alpha, beta, o, T, V, nvt, K, (int)heads,
-                       ingest_ieee(addr_bits(h0, h, scale), heads, K, V), qmax, one / qmax};
+  const bool ieee = ingest_ieee(addr_bits(h0, h, scale), heads, K, V);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return quant_mode == CK_QUANT_EXACT ? launch_decode_k<kExact>(p, heads * nvt, res_fmt, s)
-                                      : launch_decode_k<kFast>(p, heads * nvt, res_fmt, s);
+  return launch_slices(heads, nvt, kDecodeWaves * 64, [&](int64_t w0, int64_t n) {
+    const int64_t m = w0 * K * V, c = w0 * V, r = w0 * K;  // the slice's first matrix, column and row
+    const DecodeParams p{h0 + m, h + m, scale + c, static_cast<char*>(e) + m * esz, int8_res ? e_scale + c : nullptr,
+                         q + r, k + r, v + c, alpha + w0, beta + w0, o + c, T, V, nvt, K, (int)heads, ieee, qmax,
+                         one / qmax};
+    return quant_mode == CK_QUANT_EXACT ? launch_decode_k<kExact>(p, n * nvt, res_fmt, s)
+                                        : launch_decode_k<kFast>(p, n * nvt, res_fmt, s);
+  });
 }
