@@ -146,7 +146,8 @@ struct TileShape {
 };
 
 // A lane's element offset in its matrix, from its row slice and column: 32 bits, so
-// that it is one register beside a uniform base per row, and 64 in the form that heads too wide for it take.
+// that it is one register beside a uniform base per row, and 64 in the form that
+// matrices too large for it take (rows past K are not accessed: their offset may wrap).
 template <int FORM>
 using LaneOffset = std::conditional_t<FORM == kTileOne, int64_t, uint32_t>;
 

@@ -16,7 +16,8 @@ constexpr int kGroups = 32;  // column groups per workgroup (one half-wave)
 //    32) groups of 4 columns, G and the number of threads (S * G
 //    rounded up to whole waves) set per launch, so a head of any V >= 4 wastes
 //    only the last wave's rest.
-//  kTileOne: 32 single columns, for V < 4 and V > 2^21.
+//  kTileOne: 32 single columns, for V < 4 and where the others' lane offsets do
+//    not reach: 2^32 elements (KP V) with 32-bit ones, 2^30 columns otherwise.
 // The tiles of a matrix are of equal width (a multiple of 4) and the last one has
 // at least 4 columns, so its last thread can take the 4 that end with V, sharing
 // some with its neighbour in the same workgroup; the threads past S * G repeat the
@@ -28,8 +29,6 @@ enum TileForm : int { kTileFull, kTileAny, kTileOne };
 
 constexpr int max_groups(int KP) { return KP <= 128 ? 40 : 32; }
 
-constexpr int kMaxTileV = 1 << 21;
-
 struct ColTiles {
   int nvt, width;   // tiles and columns per tile (the last one: what is left)
   int groups;       // column groups per tile
@@ -40,8 +39,9 @@ struct ColTiles {
 // fp32_rows: the rows' largest elements are fp32; a tile of 24 groups or more is
 // then better left in the full form (HV=32, K=128, V=96, B=40, us, full / any: fp32
 // step 20.3 / 22.3, fp32 residual 31.8 / 32.8; fp16 21.4 / 20.3, fp8 17.3 / 15.9).
-inline ColTiles col_tiles(int V, int KP, bool fp32_rows) {
-  const int cpt = V >= 4 && V <= kMaxTileV ? 4 : 1;
+inline ColTiles col_tiles(int V, int KP, bool fp32_rows, bool offsets32) {
+  const bool reach = offsets32 ? (int64_t)KP * V < (int64_t)1 << 32 : V <= 1 << 30;
+  const int cpt = V >= 4 && reach ? 4 : 1;
   const int all = (V + cpt - 1) / cpt;  // column groups
   const int rest = V % (kGroups * 4);
   const bool full = rest == 0 || (fp32_rows && V % 4 == 0 && rest >= 96);

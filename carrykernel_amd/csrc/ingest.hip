@@ -411,7 +411,7 @@ template <int FORM>
 void launch_cols_form(const ColsParams& p, int KP, int64_t M, bool ieee, hipStream_t s) {
   if (KP != p.K) launch_cols<FORM, true, true>(p, KP, M, s);
   else if (ieee) launch_cols<FORM, false, true>(p, KP, M, s);
-  else launch_cols<FORM, false, false>(p, KP, M, s);  // V % 4 == 0: kTileOne for a V past kMaxTileV
+  else launch_cols<FORM, false, false>(p, KP, M, s);  // V % 4 == 0: kTileOne past 2^30 columns
 }
 
 // K above 256: one thread per (matrix, V-column); consecutive threads take
@@ -513,7 +513,7 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const uintptr_t bits = qs::addr_bits(x, codes, scale);
   const int KP = K <= 256 ? qs::padded_k(K) : 0;
-  const qs::ColTiles tiles = qs::col_tiles(V, KP, true);
+  const qs::ColTiles tiles = qs::col_tiles(V, KP, true, false);
   if (K <= 256) {
     const bool ieee = qs::ingest_ieee(bits, M, K, V);
     return launch_slices(M, tiles.nvt, qs::tile_threads(tiles, KP <= 128 ? 8 : 16), [&](int64_t m0, int64_t n) {

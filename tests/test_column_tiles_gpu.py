@@ -77,7 +77,7 @@ def test_step(K, V):
 
 
 def test_very_wide_head():
-    """V past the 32-bit lane offsets' limit takes the one-column form."""
+    """A ragged head of two million columns."""
     B, HV, K, V = 1, 1, 2, (1 << 21) + 3
     g = torch.Generator().manual_seed(1)
     h0 = torch.randn(B, HV, K, V, generator=g) * 0.1
@@ -99,3 +99,33 @@ def test_wide_ragged_heads(K, V):
     """Heads whose columns once left the last tile a single ragged group, in place
     and out of place."""
     test_step(K, V)
+
+
+@pytest.mark.parametrize("K,V", [(256, (1 << 24) - 4), (1, (1 << 28) + 4)])
+def test_offsets_around_32_bits(K, V):
+    """The largest matrix with 32-bit lane offsets, and one past it (one column
+    per thread): the columns at both ends as in a small head of their own."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    at = torch.cat([torch.arange(9), torch.arange(V // 2, V // 2 + 9), torch.arange(V - 9, V)]).cuda()
+    cols = lambda t: t[..., at].contiguous()  # noqa: E731
+    h = torch.randint(-127, 128, (1, 1, K, V), generator=g, device="cuda", dtype=torch.int8)
+    e = torch.randint(0, 100, (1, 1, K, V), generator=g, device="cuda", dtype=torch.uint8)
+    scale, v = torch.rand(1, 1, V, generator=g, device="cuda"), torch.randn(1, 1, V, generator=g, device="cuda")
+    x = [torch.randn(1, 1, K, device="cuda") * K ** -0.5 for _ in range(2)]
+    gates = [torch.full((1, 1), 0.9, device="cuda"), torch.full((1, 1), 0.5, device="cuda")]
+    fp8 = torch.float8_e5m2
+    got = sq.gdn_quant_step_fused(h, scale, e.view(fp8), None, *x, v, *gates, res_fmt=sq.RES_FP8)
+    ref = sq.gdn_quant_step_fused(cols(h), cols(scale), cols(e).view(fp8), None, *x, cols(v), *gates,
+                                  res_fmt=sq.RES_FP8)
+    for a, b in zip(got[:4], ref[:4]):
+        a, b = (t.view(torch.uint8) if t.dtype == fp8 else t for t in (a, b))
+        assert torch.equal(cols(a), b)
+    del got, e
+    hf = h.float()
+    got, o = sq.gdn_step_fused_fp32(hf, *x, v, *gates)
+    ref, o_ref = sq.gdn_step_fused_fp32(cols(hf), *x, cols(v), *gates)
+    assert torch.equal(cols(got), ref) and torch.equal(cols(o), o_ref)
+    del got
+    codes, s, _, _ = sq.init_quant_state(hf)
+    c_ref, s_ref, _, _ = sq.init_quant_state(cols(hf))
+    assert torch.equal(cols(codes), c_ref) and torch.equal(cols(s), s_ref)

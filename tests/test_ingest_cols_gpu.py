@@ -69,15 +69,17 @@ def test_infinities_and_huge_values(K, V):
     assert torch.equal(codes[:, :, cols], ref[:, :, cols])
 
 
-def test_very_wide_matrix():
-    """V past the four-column tiles' limit, a multiple of 4, aligned, K a power
-    of two: one column per thread in the non-IEEE arithmetic."""
-    K, V = 16, (1 << 21) + 4
-    g = torch.Generator(device="cuda").manual_seed(5)
-    x = torch.randn(K, V, generator=g, device="cuda") * 0.3
-    codes, scale = _expect(x, 127.0)
+@pytest.mark.parametrize("V", [(1 << 21) + 4, 1 << 28])
+def test_very_wide_matrix(V, K=16):
+    """Aligned, V % 4 == 0 and K a power of two (the non-IEEE arithmetic), up to
+    2^32 elements: columns of both ends and the middle as torch quantizes them."""
+    x = torch.empty(K, V, device="cuda").normal_(std=0.3, generator=torch.Generator(device="cuda").manual_seed(5))
+    at = torch.cat([torch.arange(40), torch.arange(V // 2, V // 2 + 40), torch.arange(V - 40, V)]).cuda()
+    cols = lambda t: t[..., at].contiguous()  # noqa: E731
+    codes, scale = _expect(cols(x), 127.0)
     got = sq.per_v_channel_quantize(x)
     for name, a, b in zip(("codes", "scale", "deq"), got, (codes, scale, codes.float() * scale[None, :])):
-        assert torch.equal(a, b), name
+        assert torch.equal(cols(a), b), name
+    del got
     c, s, e, es = sq.init_quant_state(x[None, None], res_fmt=sq.RES_INT8)
-    assert torch.equal(c[0, 0], codes) and torch.equal(s[0, 0], scale) and not e.any() and not es.any()
+    assert torch.equal(cols(c)[0, 0], codes) and torch.equal(cols(s)[0, 0], scale) and not e.any() and not es.any()
