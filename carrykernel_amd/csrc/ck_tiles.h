@@ -36,15 +36,34 @@ struct ColTiles {
   TileForm form;
 };
 
-// fp32_rows: the rows' largest elements are fp32; a tile of 24 groups or more is
-// then better left in the full form (HV=32, K=128, V=96, B=40, us, full / any: fp32
-// step 20.3 / 22.3, fp32 residual 31.8 / 32.8; fp16 21.4 / 20.3, fp8 17.3 / 15.9).
-inline ColTiles col_tiles(int V, int KP, bool fp32_rows, bool offsets32) {
-  const bool reach = offsets32 ? (int64_t)KP * V < (int64_t)1 << 32 : V <= 1 << 30;
+// Whether tiles of 32 whole groups are the better split of a V that is a multiple
+// of 4, the last tile's idle lanes notwithstanding. fp32_rows: the rows' largest
+// elements are fp32. Steps, us, full / any:
+//  * V > 160: two or more tiles either way, and of 33 or more groups one takes a
+//    fifth wave that is nearly empty (HV=8, K=128, V=516, B=63: int8 43.7 / 56.9,
+//    fp16 51.7 / 62.9; V=192, B=170: int8 32.4 / 35.2).
+//  * 96 < V < 128: four waves either way (K=256, V=100, B=163: int8 39.5 / 46.0);
+//    V = 96 is three waves of any (HV=32, K=128, B=40: fp32 step 20.3 / 22.3, fp32
+//    residual 31.8 / 32.8; fp16 21.4 / 20.3, fp8 17.3 / 15.9).
+//  * 128 < V <= 160: two tiles of four waves against one of five (K <= 128). From
+//    K = 128 that is better with the smaller rows only (V=132, B=248: int8 42.1 /
+//    47.5, fp32 step 62.9 / 44.4; K=64, B=496: int8 43.5 / 33.8).
+// The ingest holds fewer registers, so its fifth wave costs nothing (K=128, V=132:
+// any in 0.79 of full's time, 260 0.98, 516 1.00).
+inline bool full_tiles(int V, int KP, bool fp32_rows, bool ingest) {
+  const int rest = V % (kGroups * 4);
+  if (rest == 0) return true;
+  if (V % 4 != 0) return false;
+  if (ingest) return rest >= 96;
+  return V > 160 || rest > 96 || (rest == 96 && fp32_rows) || (V > 128 && KP >= 128 && !fp32_rows);
+}
+
+// ingest: the column ingest, whose lane offsets have 64 bits (a step's: 32).
+inline ColTiles col_tiles(int V, int KP, bool fp32_rows, bool ingest) {
+  const bool reach = ingest ? V <= 1 << 30 : (int64_t)KP * V < (int64_t)1 << 32;
   const int cpt = V >= 4 && reach ? 4 : 1;
   const int all = (V + cpt - 1) / cpt;  // column groups
-  const int rest = V % (kGroups * 4);
-  const bool full = rest == 0 || (fp32_rows && V % 4 == 0 && rest >= 96);
+  const bool full = full_tiles(V, KP, fp32_rows, ingest);
   const bool any = cpt == 4 && !full;
   int groups = kGroups;
   int nvt = (all + groups - 1) / groups;

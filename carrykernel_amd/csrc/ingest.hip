@@ -513,7 +513,7 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const uintptr_t bits = qs::addr_bits(x, codes, scale);
   const int KP = K <= 256 ? qs::padded_k(K) : 0;
-  const qs::ColTiles tiles = qs::col_tiles(V, KP, true, false);
+  const qs::ColTiles tiles = qs::col_tiles(V, KP, true, true);
   if (K <= 256) {
     const bool ieee = qs::ingest_ieee(bits, M, K, V);
     return launch_slices(M, tiles.nvt, qs::tile_threads(tiles, KP <= 128 ? 8 : 16), [&](int64_t m0, int64_t n) {

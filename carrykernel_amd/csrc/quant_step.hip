@@ -468,7 +468,7 @@ extern "C" int ck_gdn_quant_step(const int8_t* h_in, const float* scale_in, cons
   p.e_scale_out = e_scale_out;
   p.HV = HV;
   p.V = V;
-  p.tiles = col_tiles(V, padded_k(K), res_fmt == CK_RES_FP32, true);
+  p.tiles = col_tiles(V, padded_k(K), res_fmt == CK_RES_FP32, false);
   p.K = K;
   volatile float one = 1.0f;
   p.qmax = qmax;
@@ -491,7 +491,7 @@ extern "C" int ck_gdn_fp32_step(const float* h_in, const float* q, const float* 
   if (!h_in || !q || !k || !v || !alpha || !beta || !o || !h_out) return fail(CK_EINVAL, "null pointer argument");
   const uintptr_t bits = addr_bits(h_in, q, k, v, alpha, beta, o, h_out);
   if (bits & 3) return fail(CK_EINVAL, "fp32 tensors must be 4-byte aligned");
-  Fp32Params p{h_in, q, k, v, alpha, beta, o, h_out, V, col_tiles(V, padded_k(K), true, true), K};
+  Fp32Params p{h_in, q, k, v, alpha, beta, o, h_out, V, col_tiles(V, padded_k(K), true, false), K};
   const int64_t grid = (int64_t)B * HV * p.tiles.nvt;
   if (grid > 0x7fffffff) return fail(CK_EUNSUPPORTED, "grid too large");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -101,6 +101,13 @@ def test_wide_ragged_heads(K, V):
     test_step(K, V)
 
 
+@pytest.mark.parametrize("K", [16, 128, 256])
+@pytest.mark.parametrize("V", [100, 132, 164, 192, 260])
+def test_full_tiles_of_a_ragged_head(K, V):
+    """V a multiple of 4 whose last tile of whole groups has idle lanes."""
+    test_step(K, V)
+
+
 @pytest.mark.parametrize("K,V", [(256, (1 << 24) - 4), (1, (1 << 28) + 4)])
 def test_offsets_around_32_bits(K, V):
     """The largest matrix with 32-bit lane offsets, and one past it (one column
