@@ -61,13 +61,15 @@ __device__ __forceinline__ void swap_pieces(u32x4& a, u32x4& b, bool bit) {
 // bf16 rows are cached, fp32 ones stream (us, cached / streaming loads: bf16 K=128
 // B=64 24.5 / 30.3, B=128 55.9 / 56.3; fp32 K=128 B=8 9.3 / 7.8, B=64 54.5 / 50.8,
 // B=128 109 / 98; cached stores bf16 B=64 23.2, fp32 no change).
-template <bool BF16>
+// fp32 rows whose lanes take their own bytes (K = 16 and 32: an instruction touches
+// a quarter of each line) are cached too.
+template <bool CACHED>
 __device__ __forceinline__ u32x4 ld_state(const int8_t* p) {
-  return BF16 ? ld_at<u32x4>(p, 0u) : ld_stream16(p);
+  return CACHED ? ld_at<u32x4>(p, 0u) : ld_stream16(p);
 }
-template <bool BF16>
+template <bool CACHED>
 __device__ __forceinline__ void st_state(int8_t* p, u32x4 v) {
-  if constexpr (BF16) st_at<u32x4>(p, 0u, v);
+  if constexpr (CACHED) st_at<u32x4>(p, 0u, v);
   else st_stream16(p, v);
 }
 
@@ -85,6 +87,7 @@ template <int LPR, bool BF16>
 struct ChunkMap {
   static constexpr bool kSwap = LPR >= 4;
   static constexpr bool kEight = !BF16 && LPR >= 8;
+  static constexpr bool kCached = BF16 || !kSwap;
 
   __device__ static __forceinline__ uint32_t piece_off(int c, int w) {  // byte offset in the row
     if constexpr (!kSwap) return (uint32_t)(c * kPieces<BF16> + w) * 16u;
@@ -166,7 +169,7 @@ __device__ __forceinline__ void load_fitem(const PackedParams& p, const ItemCoor
     const uint32_t r = (uint32_t)min(row0 + i * L::RPI, p.V - 1) & keep;
 #pragma unroll
     for (int w = 0; w < kPieces<BF16>; ++w)
-      R.sw[i][w] = ld_state<BF16>(sbase + ((r * (K * SB) + M::piece_off(c, w)) & keep));
+      R.sw[i][w] = ld_state<M::kCached>(sbase + ((r * (K * SB) + M::piece_off(c, w)) & keep));
     R.vv[i] = load_act_raw<ESZ>(vbase, r * ESZ);
   }
   const char* qbase = mrow + (int64_t)pd::fdiv((uint32_t)hv, p.div_grp) * K * ESZ;
@@ -266,7 +269,7 @@ __device__ __forceinline__ void process_fitem(const PackedParams& p, const ItemC
     if (r < p.V) {
       if (c == 0) store_act_at(obase, (uint32_t)r, odt, o);
 #pragma unroll
-      for (int w = 0; w < kPieces<BF16>; ++w) st_state<BF16>(sbase + ((uint32_t)r * (K * SB) + M::piece_off(c, w)), out[w]);
+      for (int w = 0; w < kPieces<BF16>; ++w) st_state<M::kCached>(sbase + ((uint32_t)r * (K * SB) + M::piece_off(c, w)), out[w]);
     }
   }
 }
