@@ -62,7 +62,8 @@ __device__ __forceinline__ void swap_pieces(u32x4& a, u32x4& b, bool bit) {
 // B=64 24.5 / 30.3, B=128 55.9 / 56.3; fp32 K=128 B=8 9.3 / 7.8, B=64 54.5 / 50.8,
 // B=128 109 / 98; cached stores bf16 B=64 23.2, fp32 no change).
 // fp32 rows whose lanes take their own bytes (K = 16 and 32: an instruction touches
-// a quarter of each line) are cached too.
+// a quarter of each line) are cached too (HV=32, B=200, us, streaming / cached: K=32
+// V=128 77.2 / 42.0, V=200 125.6 / 59.0; K=16 V=128 46.1 / 25.7).
 template <bool CACHED>
 __device__ __forceinline__ u32x4 ld_state(const int8_t* p) {
   return CACHED ? ld_at<u32x4>(p, 0u) : ld_stream16(p);
@@ -150,9 +151,10 @@ template <int K, int RPL, int WAVES>
 using FLayout = pd::Layout<K, RPL, WAVES, pd::kResidInt8, false>;
 
 // All loads of one item; a dead item's collapse onto the first bytes of slot 0
-// (see pd::load_item); rows past V re-read row V-1.
-template <int K, int RPL, int WAVES, bool BF16, int ACT>
-__device__ __forceinline__ void load_fitem(const PackedParams& p, const ItemCoord& ic, int row0, int c,
+// (see pd::load_item); rows past V re-read row V-1, where SHORT leaves
+// out an instruction (rows from wave_row on) that has no other.
+template <int K, int RPL, int WAVES, bool BF16, int ACT, bool SHORT>
+__device__ __forceinline__ void load_fitem(const PackedParams& p, const ItemCoord& ic, int wave_row, int row0, int c,
                                            FloatItemRegs<RPL, FLayout<K, RPL, WAVES>::QKT, BF16>& R) {
   using L = FLayout<K, RPL, WAVES>;
   using M = ChunkMap<L::LPR, BF16>;
@@ -166,6 +168,7 @@ __device__ __forceinline__ void load_fitem(const PackedParams& p, const ItemCoor
   const char* vbase = mrow + (2 * (int64_t)p.H * K + (int64_t)hv * p.V) * ESZ;
 #pragma unroll
   for (int i = 0; i < RPL; ++i) {
+    if (SHORT && wave_row + i * L::RPI >= p.V) break;
     const uint32_t r = (uint32_t)min(row0 + i * L::RPI, p.V - 1) & keep;
 #pragma unroll
     for (int w = 0; w < kPieces<BF16>; ++w)
@@ -181,9 +184,9 @@ __device__ __forceinline__ void load_fitem(const PackedParams& p, const ItemCoor
   }
 }
 
-template <int K, int RPL, int WAVES, bool BF16, int ACT>
-__device__ __forceinline__ void process_fitem(const PackedParams& p, const ItemCoord& ic, int row0, int c, float alpha,
-                                              float beta, FloatItemRegs<RPL, FLayout<K, RPL, WAVES>::QKT, BF16>& R,
+template <int K, int RPL, int WAVES, bool BF16, int ACT, bool SHORT>
+__device__ __forceinline__ void process_fitem(const PackedParams& p, const ItemCoord& ic, int wave_row, int row0,
+                                              int c, float alpha, float beta, FloatItemRegs<RPL, FLayout<K, RPL, WAVES>::QKT, BF16>& R,
                                               float (*s_qk)[2 * K]) {
   using L = FLayout<K, RPL, WAVES>;
   using M = ChunkMap<L::LPR, BF16>;
@@ -209,6 +212,7 @@ __device__ __forceinline__ void process_fitem(const PackedParams& p, const ItemC
   int8_t* sbase = p.state + (ic.slot * p.stride_state + (int64_t)ic.hv * p.V * K) * SB;
 #pragma unroll
   for (int i = 0; i < RPL; ++i) {
+    if (SHORT && wave_row + i * L::RPI >= p.V) break;
     const int r = row0 + i * L::RPI;
     asm volatile("" ::: "memory");  // re-read k, q from LDS for this row
     float kk[16], qq[16], h[16];
@@ -275,8 +279,11 @@ __device__ __forceinline__ void process_fitem(const PackedParams& p, const ItemC
 }
 
 // One item per workgroup; the launch geometry in preloaded arguments (see
-// pd::packed_decode_single_kernel).
-template <int K, int RPL, int WAVES, bool BF16, int ACT>
+// pd::packed_decode_single_kernel). SHORT: waves without a row do no row work, for
+// heads that leave a wave of their one tile empty: its re-reads of row V-1 cost
+// (HV=32, B=200, us, without / with: fp32 K=128 V=1 26.1 / 13.3, V=16 30.9 / 20.9,
+// bf16 K=128 V=16 20.2 / 14.7); with no such wave the branches do (+0-4 % at V=128).
+template <int K, int RPL, int WAVES, bool BF16, int ACT, bool SHORT>
 __global__ __launch_bounds__(WAVES * 64)
 void float_decode_kernel(const int32_t* __restrict__ idx, int items, int stride_idx, uint32_t nvt_d, uint32_t nvt_m,
                          uint32_t nvt_sh, uint32_t hv_d, uint32_t hv_m, uint32_t hv_sh, int xcd_base, uint32_t grp_m,
@@ -292,15 +299,17 @@ void float_decode_kernel(const int32_t* __restrict__ idx, int items, int stride_
   const int c = lane % L::LPR;
   const int g = lane / L::LPR;
   const ItemCoord ic = pd::xcd_item_coord<false>(p, gm, idx, nullptr, (int)blockIdx.x, xcd_base);
-  const int row0 = ic.vt * L::ROWS_WG + wave * L::ROWS_WAVE + g;
+  const int wave_row = ic.vt * L::ROWS_WG + __builtin_amdgcn_readfirstlane(wave) * L::ROWS_WAVE;
+  const int row0 = wave_row + g;
   FloatItemRegs<RPL, L::QKT, BF16> R;
-  load_fitem<K, RPL, WAVES, BF16, ACT>(p, ic, row0, c, R);
+  if constexpr (SHORT) R = {};
+  load_fitem<K, RPL, WAVES, BF16, ACT, SHORT>(p, ic, wave_row, row0, c, R);
   __builtin_amdgcn_sched_barrier(0);  // the gate inputs' loads after the item's
   const pd::GateBits gbits = pd::load_item_gate_bits(p, ic);
   pd::stage_item_gates(p, gbits, wave, lane, s_gate);
   __syncthreads();
   const float2 gab = s_gate[0];
-  process_fitem<K, RPL, WAVES, BF16, ACT>(p, ic, row0, c, gab.x, gab.y, R, s_qk);
+  process_fitem<K, RPL, WAVES, BF16, ACT, SHORT>(p, ic, wave_row, row0, c, gab.x, gab.y, R, s_qk);
 }
 
 template <int K, int RPL, bool BF16, int ACT>
@@ -326,9 +335,11 @@ int launch_fs_cfg(PackedParams p, int B, hipStream_t stream) {
   p.items = (int)items;
   p.div_nvt = pd::make_fastdiv((uint32_t)nvt);
   p.div_hv = pd::make_fastdiv((uint32_t)p.HV);
-  hipLaunchKernelGGL((float_decode_kernel<K, RPL, WAVES, BF16, ACT>), dim3((unsigned)items), dim3(WAVES * 64), 0,
-                     stream, p.idx, p.items, p.stride_idx, p.div_nvt.d, p.div_nvt.m, p.div_nvt.sh, p.div_hv.d,
-                     p.div_hv.m, p.div_hv.sh, pd::xcd_base(B, p.HV * nvt), p.div_grp.m, pd::quotient_word(p.div_grp), p);
+  auto fn = float_decode_kernel<K, RPL, WAVES, BF16, ACT, false>;
+  if (p.V <= L::ROWS_WG - L::ROWS_WAVE) fn = float_decode_kernel<K, RPL, WAVES, BF16, ACT, true>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)items), dim3(WAVES * 64), 0, stream, p.idx, p.items, p.stride_idx, p.div_nvt.d,
+                     p.div_nvt.m, p.div_nvt.sh, p.div_hv.d, p.div_hv.m, p.div_hv.sh, pd::xcd_base(B, p.HV * nvt),
+                     p.div_grp.m, pd::quotient_word(p.div_grp), p);
   return check_launch("ck_gdn_packed_decode_float_state");
 }
 
