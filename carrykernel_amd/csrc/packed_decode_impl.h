@@ -364,14 +364,16 @@ __device__ __forceinline__ void stage_qk(const PackedParams& p, const uint32_t (
 // How the masked kernel's rows are accessed: rows are p.K codes long (K is
 // p.K rounded up to a power of two, at least 16), at any byte alignment (global
 // memory takes accesses of any alignment on this target).
-//  kMaskBytes: p.K below 16 (less than a lane), byte by byte.
+//  kMaskShort: p.K below 16 (less than a lane): the lane loads the row's first and
+//    last W bytes, W the power of two that n < 2 W bytes hold, and puts them
+//    together at use; it stores as kMaskTail.
 //  kMaskLanes: p.K a multiple of 16, so a lane's 16 codes (and 8 or 16 residual
 //    bytes) are all there or all past p.K, and it loads and stores them whole.
 //  kMaskTail: any other p.K; the lane that holds the row's end loads the row's
 //    last 16 codes (8 or 16 residual bytes), which lie inside the row, and
 //    shifts the first ones out; it stores its bytes in pieces of 8, 4, 2 and 1.
 constexpr int kMaskNone = 0;
-constexpr int kMaskBytes = 1;
+constexpr int kMaskShort = 1;
 constexpr int kMaskLanes = 2;
 constexpr int kMaskTail = 3;
 
@@ -395,13 +397,39 @@ __device__ __forceinline__ void shift_right_bytes(uint32_t (&w)[2], int d) {  //
   w[0] = (uint32_t)x, w[1] = (uint32_t)(x >> 32);
 }
 
-// The first n bytes (n clamped to 0 .. 4 NW) of w, byte j from dword j / 4,
-// one byte store each (kMaskBytes).
+// kMaskShort: the n bytes of a row at p (1 <= n < 4 NW) as two pieces of W bytes,
+// in the halves of w, and the row's bytes from them. n is uniform, so the
+// branches are too.
 template <int NW>
-__device__ __forceinline__ void st_bytes_masked(int8_t* dst, const uint32_t (&w)[NW], int n) {
+__device__ __forceinline__ void ld_pieces(const int8_t* p, int n, uint32_t (&w)[NW]) {
 #pragma unroll
-  for (int j = 0; j < 4 * NW; ++j)
-    if (j < n) dst[j] = (int8_t)(w[j >> 2] >> (8 * (j & 3)));
+  for (int j = 0; j < NW; ++j) w[j] = 0u;
+  if (NW == 4 && n >= 8) {
+    const u32x2 a = ld_8_u<false>(p), b = ld_8_u<false>(p + n - 8);
+    w[0] = a.x, w[1] = a.y, w[NW - 2] = b.x, w[NW - 1] = b.y;
+  } else if (n >= 4) {
+    w[0] = *reinterpret_cast<const u32_u*>(p), w[NW / 2] = *reinterpret_cast<const u32_u*>(p + n - 4);
+  } else if (n >= 2) {
+    w[0] = *reinterpret_cast<const u16_u*>(p), w[NW / 2] = *reinterpret_cast<const u16_u*>(p + n - 2);
+  } else {
+    w[0] = *reinterpret_cast<const uint8_t*>(p);
+  }
+}
+template <int NW>
+__device__ __forceinline__ void join_pieces(uint32_t (&w)[NW], int n) {
+  if (NW == 4 && n >= 8) {
+    const uint64_t b = n == 8 ? 0u : (((uint64_t)w[NW - 1] << 32) | w[NW - 2]) >> (8 * (16 - n));
+    w[NW - 2] = (uint32_t)b, w[NW - 1] = (uint32_t)(b >> 32);
+    return;
+  }
+  const uint32_t b = w[NW / 2];
+  if (NW == 4) w[NW / 2] = 0u;
+  if (n >= 4) {
+    w[1] = n == 4 ? 0u : b >> (8 * (8 - n));
+  } else {
+    if (n == 3) w[0] |= (b >> 8) << 16;
+    w[1] = 0u;
+  }
 }
 
 // A lane's 4 NW bytes, or those of its first n that exist (kMaskTail): which
@@ -442,9 +470,7 @@ template <int RESID, int MASK>
 __device__ __forceinline__ void store_resid_masked(int8_t* dst, const uint32_t (&eb)[16], int row_bytes, int n) {
   uint32_t w[RESID == kResidInt4 ? 2 : 4];
   pack_resid<RESID>(eb, w);
-  if constexpr (MASK == kMaskBytes) {
-    st_bytes_masked(dst, w, n);
-  } else if constexpr (MASK == kMaskTail) {
+  if constexpr (MASK == kMaskTail || MASK == kMaskShort) {
     st_tail(dst, w, row_bytes, n);
   } else if (n > 0) {
     if constexpr (RESID == kResidInt4) st_stream8_u(dst, u32x2{w[0], w[1]});
@@ -532,7 +558,10 @@ __device__ __forceinline__ void process_item(const PackedParams& p, const ItemCo
     uint32_t ews[L::EW];
 #pragma unroll
     for (int j = 0; j < L::EW; ++j) ews[j] = R.ew[i][j];
-    if constexpr (MASK == kMaskTail) {
+    if constexpr (MASK == kMaskShort) {
+      join_pieces(cws, KA);
+      join_pieces(ews, RKA);
+    } else if constexpr (MASK == kMaskTail) {
       shift_right_bytes(cws, tail_shift<4>(c * 16, KA) & 15);  // lanes past the row hold zeros
       shift_right_bytes(ews, tail_shift<L::EW>(c * RKL, RKA) & (4 * L::EW - 1));
     }
@@ -612,9 +641,7 @@ __device__ __forceinline__ void process_item(const PackedParams& p, const ItemCo
     if (store) {
       const uint32_t w[4] = {pack_low_bytes(yb[0], yb[1], yb[2], yb[3]), pack_low_bytes(yb[4], yb[5], yb[6], yb[7]),
                              pack_low_bytes(yb[8], yb[9], yb[10], yb[11]), pack_low_bytes(yb[12], yb[13], yb[14], yb[15])};
-      if constexpr (MASK == kMaskBytes) {
-        st_bytes_masked<4>(sbase + (soff + (uint32_t)(i * L::RPI * KA)), w, KA - c * 16);
-      } else if constexpr (MASK == kMaskTail) {
+      if constexpr (MASK == kMaskTail || MASK == kMaskShort) {
         st_tail<4>(sbase + (soff + (uint32_t)(i * L::RPI * KA)), w, KA, KA - c * 16);
       } else if constexpr (MASK == kMaskLanes) {
         if (c * 16 < KA) st_stream16_u(sbase + (soff + (uint32_t)(i * L::RPI * KA)), u32x4{w[0], w[1], w[2], w[3]});

@@ -7,7 +7,8 @@
 // arithmetic of packed_decode_impl.h (process_item) on that padded row: the
 // lane map of KP, every value past K zero in registers, stores of the K
 // existing bytes only. A lane's codes come and go in one access of any
-// alignment (packed_decode_impl.h, kMaskLanes and kMaskTail); the activations
+// alignment, two for rows of less than a lane (packed_decode_impl.h, kMaskLanes,
+// kMaskTail and kMaskShort); the activations
 // are loaded as raw words first, the state after them, and decoded while it is
 // in flight. One item per workgroup. The bandwidth kernels cover aligned pools
 // of the power-of-two K of real models, this one every other shape.
@@ -85,24 +86,12 @@ __device__ __forceinline__ void load_item_masked(const PackedParams& p, const It
     if constexpr (!PER_HEAD) R.es_in[i] = ld_at<float>(rsb, r * 4u);
   }
   if constexpr (PER_HEAD) R.es_in[0] = p.rscale[ic.slot * p.stride_rscale + ic.hv];
-  if constexpr (MASK == kMaskBytes) {
+  if constexpr (MASK == kMaskShort) {  // one lane per row
 #pragma unroll
     for (int i = 0; i < RPL; ++i) {
-      const int64_t r = min(row0 + i * L::RPI, p.V - 1);
-      const int8_t* srow = sbase + r * K;
-      const int8_t* erow = ebase + r * RKA;
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      uint32_t e[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int k = c * 16 + j;
-        if (k < K) w[j >> 2] |= (uint32_t)(uint8_t)srow[k] << (8 * (j & 3));
-      }
-#pragma unroll
-      for (int j = 0; j < RKL; ++j) {
-        const int bidx = c * RKL + j;
-        if (bidx < RKA) e[j >> 2] |= (uint32_t)(uint8_t)erow[bidx] << (8 * (j & 3));
-      }
+      uint32_t w[4], e[L::EW];
+      ld_pieces(sbase + clamped_row_offset(row0, i * L::RPI, K, p.V), K, w);
+      ld_pieces(ebase + clamped_row_offset(row0, i * L::RPI, RKA, p.V), RKA, e);
       R.cw[i] = u32x4{w[0], w[1], w[2], w[3]};
 #pragma unroll
       for (int j = 0; j < L::EW; ++j) R.ew[i][j] = e[j];
@@ -289,7 +278,7 @@ int launch_masked_k(const PackedParams& p, int B, int resid_fmt, int per_head, i
   int launch_masked_k<KP>(const PackedParams& p, int B, int resid_fmt, int per_head, int mode,               \
                           hipStream_t s) {                                                                   \
     if (p.K % 16 == 0) return launch_masked_mode<KP, kMaskLanes>(p, B, resid_fmt, per_head, mode, s);        \
-    constexpr int kRest = KP == 16 ? kMaskBytes : kMaskTail;                                                 \
+    constexpr int kRest = KP == 16 ? kMaskShort : kMaskTail;                                                 \
     return launch_masked_mode<KP, kRest>(p, B, resid_fmt, per_head, mode, s);                                \
   }
 

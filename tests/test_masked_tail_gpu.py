@@ -74,3 +74,12 @@ def test_partly_filled_workgroups(K, V):
     """Per head (waves without a row are not launched) and per row (they skip)."""
     _run(K, V, 2, 3, qpd.RESID_INT4, True, lead=1)
     _run(K, V, 2, 3, qpd.RESID_INT8, False, lead=1)
+
+
+@pytest.mark.parametrize("K", range(1, 16))
+@pytest.mark.parametrize("per_head", [False, True])
+def test_rows_of_less_than_a_lane(K, per_head):
+    """K below 16: a row is put together from its first and last bytes."""
+    _run(K, 67, 3, 2, qpd.RESID_INT8, per_head, lead=K % 3, act=torch.bfloat16)
+    if K % 2 == 0:
+        _run(K, 67, 3, 2, qpd.RESID_INT4, per_head, mode="exact", lead=K % 5)
