@@ -201,7 +201,10 @@ int launch_masked_cfg(PackedParams p, int B, hipStream_t stream) {
 // Shapes. Per-row residual scales: 4 waves of two rows per lane from 1024 such
 // tiles on, below that (and above K = 256) of one row, which spreads a small
 // batch over more SIMDs (HV=16, V=100, K=100 int8, us, one row / two rows: B=24,
-// 768 tiles 8.1 / 8.3; B=64, 2048 tiles 15.0 / 14.3; B=128 24.9 / 23.2).
+// 768 tiles 8.1 / 8.3; B=64, 2048 tiles 15.0 / 14.3; B=128 24.9 / 23.2); one row
+// also where four waves of it cover the head, which two rows would leave to one or
+// two of them (B=64, HV=32, us, one / two: K=36 V=64 int4 exact 10.6 / 12.3, K=200
+// V=16 12.3 / 14.4, K=8 V=128 int8 8.3 / 9.3).
 // A per-head scale needs the whole head in one workgroup: at KP=64 and 128 a
 // head that four or eight waves of two rows per lane hold takes those, at
 // KP=256 sixteen (fewer registers than four rows per lane, so more workgroups
@@ -218,7 +221,7 @@ template <int KP, int RESID, bool PER_HEAD, int MODE, bool DST, int MASK>
 int launch_masked_shape(const PackedParams& p, int B, hipStream_t s) {
   constexpr int RPI = 64 / (KP / 16);
   if constexpr (!PER_HEAD) {
-    if (KP <= 256 && (int64_t)B * p.HV * ((p.V + RPI * 8 - 1) / (RPI * 8)) >= 1024)
+    if (KP <= 256 && p.V > RPI * 4 && (int64_t)B * p.HV * ((p.V + RPI * 8 - 1) / (RPI * 8)) >= 1024)
       return launch_masked_cfg<KP, 2, 4, RESID, false, MODE, DST, MASK>(p, B, s);
     return launch_masked_cfg<KP, 1, 4, RESID, false, MODE, DST, MASK>(p, B, s);
   } else {
