@@ -253,6 +253,15 @@ __global__ __launch_bounds__(256) void zero_residual_kernel(int8_t* __restrict__
   for (int64_t i = t; i < n_rscale; i += n) rscale[i] = 0.0f;
 }
 
+void launch_zero_residual(int8_t* resid, int64_t bytes, float* rscale, int64_t n_rscale, hipStream_t s) {
+  if (!resid) bytes = 0;
+  if (!rscale) n_rscale = 0;
+  if (bytes == 0 && n_rscale == 0) return;
+  const int64_t blocks = (std::max(bytes / 16, n_rscale) + 255) / 256 + 1;
+  hipLaunchKernelGGL(zero_residual_kernel, dim3((unsigned)std::min<int64_t>(blocks, 4096)), dim3(256), 0, s, resid,
+                     bytes, rscale, n_rscale);
+}
+
 // Rows shorter or longer than the tile kernel takes: one wavefront per row; lanes
 // stride over K. 16-bit
 // dtypes in their own precision (RN16 after each fp32 operation).
@@ -415,12 +424,15 @@ void launch_cols_form(const ColsParams& p, int KP, int64_t M, bool ieee, hipStre
 }
 
 // K above 256: one thread per (matrix, V-column); consecutive threads take
-// consecutive columns so every K-row access is coalesced.
+// consecutive columns so every K-row access is coalesced. The two passes over a
+// column's rows are what a small matrix waits for, so a residual is zeroed by a
+// launch of its own ([4, 8, 1024, 64], us a call: fp32 residual 345 in the second
+// pass, 251 so; dequantized values as a run-time branch of it 333, 275 as a kernel
+// of its own, 320 without the unrolling).
+template <bool DEQ>
 __global__ __launch_bounds__(256) void quantize_cols_kernel(const float* __restrict__ x, int64_t M, int K, int V,
                                                             float qmax, int8_t* __restrict__ codes,
-                                                            float* __restrict__ scale, float* __restrict__ deq,
-                                                            char* __restrict__ e, int e_bytes,
-                                                            float* __restrict__ e_scale) {
+                                                            float* __restrict__ scale, float* __restrict__ deq) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= M * V) return;
   const int64_t m = t / V;
@@ -430,17 +442,15 @@ __global__ __launch_bounds__(256) void quantize_cols_kernel(const float* __restr
   for (int j = 0; j < K; ++j) am = fmaxf(am, fabsf(xm[(int64_t)j * V]));
   const float s = fmaxf(am, kEps) / qmax;
   int8_t* cm = codes + m * K * V + c;
+  float* dm = DEQ ? deq + m * K * V + c : nullptr;
+#pragma unroll 8
   for (int j = 0; j < K; ++j) {
     const float q = fminf(fmaxf(rintf(xm[(int64_t)j * V] / s), -qmax), qmax);
     const int8_t code = (int8_t)(int)q;
-    const int64_t i = m * K * V + (int64_t)j * V + c;
     cm[(int64_t)j * V] = code;
-    if (deq) deq[i] = (float)code * s;
-    if (e)
-      for (int b = 0; b < e_bytes; ++b) e[i * e_bytes + b] = 0;
+    if constexpr (DEQ) dm[(int64_t)j * V] = (float)code * s;
   }
   scale[m * V + c] = s;
-  if (e_scale) e_scale[m * V + c] = 0.0f;
 }
 
 }  // namespace
@@ -481,12 +491,7 @@ extern "C" int ck_quantize_rows_init(const void* x, int x_dtype, int64_t stride_
     return fail(CK_EINVAL, "float64 rows must be 8-byte aligned");
   const int64_t grid = (rows + 3) / 4;
   if (grid > 0x7fffffff) return fail(CK_EUNSUPPORTED, "too many rows");
-  if (resid || rscale) {
-    const int64_t bytes = resid ? rows * resid_row_bytes : 0;
-    const int64_t blocks = (std::max(bytes / 16, n_rscale) + 255) / 256 + 1;
-    hipLaunchKernelGGL(zero_residual_kernel, dim3((unsigned)std::min<int64_t>(blocks, 4096)), dim3(256), 0, s, resid,
-                       bytes, rscale, n_rscale);
-  }
+  launch_zero_residual(resid, rows * resid_row_bytes, rscale, n_rscale, s);
   if (x_dtype == CK_DTYPE_F64)
     hipLaunchKernelGGL(quantize_rows_f64_kernel, dim3((unsigned)grid), dim3(256), 0, s, static_cast<const double*>(x),
                        stride_row, rows, K, (double)qmax, codes, scale);
@@ -530,7 +535,12 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   }
   const int64_t grid = (M * V + 255) / 256;
   if (grid > 0x7fffffff) return fail(CK_EUNSUPPORTED, "too many columns");
-  hipLaunchKernelGGL(quantize_cols_kernel, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes, scale, deq,
-                     static_cast<char*>(e), e_bytes, e_scale);
+  launch_zero_residual(static_cast<int8_t*>(e), M * K * V * e_bytes, e_scale, M * V, s);
+  if (deq)
+    hipLaunchKernelGGL(quantize_cols_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes, scale,
+                       deq);
+  else
+    hipLaunchKernelGGL(quantize_cols_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes,
+                       scale, deq);
   return check_launch("ck_quantize_cols");
 }
