@@ -78,6 +78,26 @@ inline ColTiles col_tiles(int V, int KP, bool fp32_rows, bool ingest) {
                   cpt == 1 ? kTileOne : full ? kTileFull : kTileAny};
 }
 
+// Whether the column ingest is faster with one thread per column than with a
+// workgroup per matrix: many matrices, each too small for one. A workgroup costs
+// about 0.5 ns (KP = 16) to 5 ns (256) of the chip's time however few columns it
+// has; a column's thread K row accesses one after another, 0.4 us each, and lines
+// that its neighbours use only while they stay in L2. us, workgroups / threads:
+//  * M: [1, 1] 64 matrices 2.4 / 2.2, 4096 3.9 / 2.4, 262144 108 / 2.9; [8, 4] 4096
+//    4.5 / 4.1; [16, 3] 4096 4.6 / 6.8, 32768 20.8 / 8.3; [128, 1] 4096 13.7 / 62,
+//    32768 80 / 63.
+//  * K <= 16: 65535 of [8, 32] 32 / 28, 262144 of it 126 / 151, of [16, 12] 118 / 89,
+//    of [16, 16] 129 / 140.
+//  * K <= 32: 65535 of [32, 6] 50 / 44, 262144 of [32, 8] 193 / 163, [32, 12] 206 / 242.
+//  * above: 65535 of [64, 3] 91 / 63, [100, 4] 143 / 93, [128, 3] 158 / 129, [128, 5]
+//    157 / 175; 262144 of [64, 1] 351 / 529.
+inline bool few_columns(int64_t M, int K, int V) {
+  if (K > 2 && M < (K <= 16 ? 512 * K : 16384)) return false;
+  if (K <= 16) return K * (int64_t)V <= (M <= 1 << 17 ? 256 : 224);
+  if (K <= 32) return V <= 8;
+  return V <= 4 && M <= 1 << 17;
+}
+
 // Threads of a workgroup with S slices.
 inline int tile_threads(const ColTiles& t, int S) { return (t.groups * S + 63) / 64 * 64; }
 

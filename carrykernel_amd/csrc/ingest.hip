@@ -423,16 +423,15 @@ void launch_cols_form(const ColsParams& p, int KP, int64_t M, bool ieee, hipStre
   else launch_cols<FORM, false, false>(p, KP, M, s);  // V % 4 == 0: kTileOne past 2^30 columns
 }
 
-// K above 256: one thread per (matrix, V-column); consecutive threads take
-// consecutive columns so every K-row access is coalesced. The two passes over a
-// column's rows are what a small matrix waits for, so a residual is zeroed by a
-// launch of its own ([4, 8, 1024, 64], us a call: fp32 residual 345 in the second
-// pass, 251 so; dequantized values as a run-time branch of it 333, 275 as a kernel
-// of its own, 320 without the unrolling).
-template <bool DEQ>
+// K above 256, and many small matrices (few_columns): one thread per (matrix,
+// V-column); consecutive threads take consecutive columns so every K-row access is
+// coalesced. The two passes over a column's rows are what a small matrix waits
+// for, and a narrow one's rows lie apart, so a residual and the dequantized values
+// are written by launches of their own (us a call: [4, 8, 1024, 64] int8 residual
+// 342 in the second pass, 286 so).
 __global__ __launch_bounds__(256) void quantize_cols_kernel(const float* __restrict__ x, int64_t M, int K, int V,
                                                             float qmax, int8_t* __restrict__ codes,
-                                                            float* __restrict__ scale, float* __restrict__ deq) {
+                                                            float* __restrict__ scale) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= M * V) return;
   const int64_t m = t / V;
@@ -442,15 +441,26 @@ __global__ __launch_bounds__(256) void quantize_cols_kernel(const float* __restr
   for (int j = 0; j < K; ++j) am = fmaxf(am, fabsf(xm[(int64_t)j * V]));
   const float s = fmaxf(am, kEps) / qmax;
   int8_t* cm = codes + m * K * V + c;
-  float* dm = DEQ ? deq + m * K * V + c : nullptr;
-#pragma unroll 8
   for (int j = 0; j < K; ++j) {
     const float q = fminf(fmaxf(rintf(xm[(int64_t)j * V] / s), -qmax), qmax);
-    const int8_t code = (int8_t)(int)q;
-    cm[(int64_t)j * V] = code;
-    if constexpr (DEQ) dm[(int64_t)j * V] = (float)code * s;
+    cm[(int64_t)j * V] = (int8_t)(int)q;
   }
   scale[m * V + c] = s;
+}
+
+// deq = code * scale of those: a workgroup takes `per` of the M K rows at a time
+// (1024 elements, or one row).
+__global__ __launch_bounds__(256) void dequantize_cols_kernel(const int8_t* __restrict__ codes,
+                                                              const float* __restrict__ scale, int64_t rows, int K,
+                                                              int V, int per, float* __restrict__ deq) {
+  for (int64_t r0 = (int64_t)blockIdx.x * per; r0 < rows; r0 += (int64_t)gridDim.x * per) {
+    const int64_t m0 = r0 / K;
+    const uint32_t k0 = (uint32_t)(r0 - m0 * K), n = (uint32_t)min((int64_t)per, rows - r0) * (uint32_t)V;
+    for (uint32_t i = threadIdx.x; i < n; i += 256) {
+      const uint32_t row = i / (uint32_t)V, c = i - row * (uint32_t)V;
+      deq[r0 * V + i] = (float)codes[r0 * V + i] * scale[(m0 + (k0 + row) / (uint32_t)K) * V + c];
+    }
+  }
 }
 
 }  // namespace
@@ -519,8 +529,8 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   const uintptr_t bits = qs::addr_bits(x, codes, scale);
   const int KP = K <= 256 ? qs::padded_k(K) : 0;
   const qs::ColTiles tiles = qs::col_tiles(V, KP, true, true);
-  if (K <= 256) {
-    const bool ieee = qs::ingest_ieee(bits, M, K, V);
+  const bool ieee = qs::ingest_ieee(bits, M, K, V);
+  if (K <= 256 && !(ieee && qs::few_columns(M, K, V))) {
     return launch_slices(M, tiles.nvt, qs::tile_threads(tiles, KP <= 128 ? 8 : 16), [&](int64_t m0, int64_t n) {
       const int64_t i = m0 * K * V, c = m0 * V;  // the slice's first matrix and column
       const ColsParams p{x + i, V, tiles, K, qmax, codes + i, scale + c, deq ? deq + i : nullptr,
@@ -536,11 +546,11 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   const int64_t grid = (M * V + 255) / 256;
   if (grid > 0x7fffffff) return fail(CK_EUNSUPPORTED, "too many columns");
   launch_zero_residual(static_cast<int8_t*>(e), M * K * V * e_bytes, e_scale, M * V, s);
-  if (deq)
-    hipLaunchKernelGGL(quantize_cols_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes, scale,
-                       deq);
-  else
-    hipLaunchKernelGGL(quantize_cols_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes,
-                       scale, deq);
+  hipLaunchKernelGGL(quantize_cols_kernel, dim3((unsigned)grid), dim3(256), 0, s, x, M, K, V, qmax, codes, scale);
+  if (deq) {
+    const int64_t rows = M * K, per = std::max(1024 / V, 1), blocks = (rows + per - 1) / per;
+    hipLaunchKernelGGL(dequantize_cols_kernel, dim3((unsigned)std::min<int64_t>(blocks, 1 << 16)), dim3(256), 0, s,
+                       codes, scale, rows, K, V, (int)per, deq);
+  }
   return check_launch("ck_quantize_cols");
 }

@@ -83,3 +83,21 @@ def test_very_wide_matrix(V, K=16):
     del got
     c, s, e, es = sq.init_quant_state(x[None, None], res_fmt=sq.RES_INT8)
     assert torch.equal(cols(c)[0, 0], codes) and torch.equal(cols(s)[0, 0], scale) and not e.any() and not es.any()
+
+
+@pytest.mark.parametrize("M,K,V", [(3, 1, 256), (3, 2, 127), (4096, 4, 7), (8192, 16, 16), (8192, 16, 17),
+                                   (16384, 17, 6), (16384, 32, 9), (16384, 100, 4), (16384, 256, 3), (65536, 128, 4)])
+def test_many_small_matrices(M, K, V):
+    """One thread per column up to a few columns, a workgroup per matrix above."""
+    x = torch.randn(M, K, V, generator=torch.Generator(device="cuda").manual_seed(K + V), device="cuda")
+    x[1], x[2, 0, 0] = 0.0, float("inf")
+    codes, scale = _expect(x, 127.0)
+    got = sq.per_v_channel_quantize(x)
+    ok = torch.ones_like(scale, dtype=torch.bool)
+    ok[2, 0] = False   # the infinity's column: a scale of inf, its other codes 0
+    assert torch.equal(got[1], scale) and torch.equal(got[0].mT[ok], codes.mT[ok])
+    assert torch.equal(got[2].mT[ok], (codes.float() * scale[:, None, :]).mT[ok]) and not got[0][2, 1:, 0].any()
+    for fmt in (sq.RES_FP32, sq.RES_FP16, sq.RES_FP8, sq.RES_INT8):
+        c, s, e, es = sq.init_quant_state(x, res_fmt=fmt)
+        assert torch.equal(c, got[0]) and torch.equal(s, scale) and not e.float().any()
+        assert (es is None) == (fmt != sq.RES_INT8) and (es is None or not es.any())
