@@ -43,30 +43,37 @@ __device__ __forceinline__ float round16_rt(int dt, float x) {
   return dt == kBF16 ? round16<kBF16>(x) : dt == kF16 ? round16<kF16>(x) : x;
 }
 
-// Rows of K elements, a wave several rows at a time: a lane takes 16 bytes of a
-// row (EPL elements, one access of any alignment), W lanes cover a row, U rows
-// per lane are in flight, and the W lanes take the row amax among them. In the
-// same pass, where asked for: a zero residual of rk bytes per row and zero
-// scales, which took the caller two launches and, with those that cleared the
-// codes and scales before they were written, a pass over the pool.
-// HBM is the bound. ANY: K is p.K and no multiple of EPL need be; the last lane
-// then takes the row's last EPL elements, some of them its neighbour's too (the
-// same codes). Two arithmetics, equal on finite values:
-//  * K a power of two from 16 to 256, 16-byte aligned: each element through
-//    RN(1/s) with Markstein's correction (ck_quant.h, EXACT mode), the correctly
-//    rounded quotient. |x / s| <= qmax (1 + 2^-23) < qmax + 1/2 since s >= RN(amax
-//    / qmax), so no code exceeds qmax and the clamp of the reference never
-//    binds. The amax keeps a 16-element chunk of NaNs as NaN.
-//  * ANY: IEEE quotients and the clamp (infinities, scales that are no normal
-//    number), NaN codes 0 and NaNs no part of the amax.
+// Rows of K elements, a wave several rows at a time, in one pass: codes, scales
+// and, where asked for, a zero residual of rk bytes per row and zero scales, which
+// took the caller two launches and, with those that cleared the codes and scales
+// before they were written, a pass over the pool. Two kernels, equal on finite
+// values:
+//  * K a power of two from 16 to 256, 16-byte aligned (quantize_rows16_kernel): 16
+//    elements per lane, each through RN(1/s) with Markstein's correction (ck_quant.h,
+//    EXACT mode), the correctly rounded quotient. |x / s| <= qmax (1 + 2^-23) < qmax +
+//    1/2 since s >= RN(amax / qmax), so no code exceeds qmax and the clamp of the
+//    reference never binds. The amax keeps a 16-element chunk of NaNs as NaN.
+//  * any other (quantize_rows_tile_kernel), 16 bytes of a row per lane in one access
+//    of any alignment, four rows in flight: IEEE quotients and the clamp (infinities,
+//    scales that are no normal number), NaN codes 0 and NaNs no part of the amax.
 // 16-bit dtypes in their own precision: RN16 after every fp32 operation.
-// Without ANY the lanes of a pair (fp32: quad) exchange codes of their U rows, so
-// that each stores 16 bytes of one row: a wave's 8 or 4 bytes a lane took 21.1 us.
-// Measured, init_quantized_state of a bf16 [64, 32, 128, 128] with an int4
-// residual (118 MB): 32.4 -> 19.6 us a call (6.0 TB/s; 26.7 with bf16 rounded by
-// integer operations); before, four fills and a kernel whose lanes loaded 16
-// elements each in two accesses. [32, 32, 100, 100] int8: fp32 40.8 -> 14.7, bf16
-// 42.1 -> 15.6 (two passes of one wave per row before).
+// HBM bounds large fp32 states (5.6 TB/s at 257 slots of [32, 128, 128]), HBM and
+// about 12 VALU operations an element 16-bit ones (6.6 TB/s). Row-level work is done
+// once per 16 elements: 4 or 8 elements per lane in one access each, with the codes
+// exchanged into 16-byte stores, were slower (us, so / now: 257 slots bf16 70.2 /
+// 60.6, fp16 67.4 / 60.3, fp32 123.0 / 121.0; 8 slots bf16 6.0 / 4.2), and so were
+// whole lines per access with the pieces swapped between lanes (257 slots bf16 64.7,
+// fp32 124.0): the loads are cached, the next instruction's bytes L2 hits.
+// init_quantized_state of a bf16 [64, 32, 128, 128] with an int4 residual (118 MB),
+// four fills and a kernel / one pass: 35.1 / 22.0 us a call. [32, 32, 100, 100] int8:
+// fp32 40.8 -> 14.7, bf16 42.1 -> 15.6 (two passes of one wave per row before).
+struct RowsInit {
+  int8_t* resid;    // or null
+  int rk;           // residual bytes per row
+  float* rscale;    // or null
+  int64_t n_rscale;
+};
+
 struct RowsParams {
   const char* x;
   int64_t stride_row_bytes, rows;
@@ -74,40 +81,132 @@ struct RowsParams {
   float qmax;
   int8_t* codes;
   float* scale;
-  int8_t* resid;    // or null
-  int rk;           // residual bytes per row
-  float* rscale;    // or null
-  int64_t n_rscale;
+  RowsInit init;
 };
 
-// Unsigned maximum from groups of N0 lanes (already reduced) to groups of N.
-template <int N0, int N>
-__device__ __forceinline__ float group_max_from(float x) {
-  uint32_t u = __float_as_uint(x);
-  if constexpr (N0 < 2 && N >= 2) u = max(u, dpp_u<kDppQuadXor1>(u));
-  if constexpr (N0 < 4 && N >= 4) u = max(u, dpp_u<kDppQuadXor2>(u));
-  if constexpr (N0 < 8 && N >= 8) u = max(u, dpp_u<kDppRowHalfMirror>(u));
-  if constexpr (N0 < 16 && N >= 16) u = max(u, dpp_u<kDppRowMirror>(u));
-  if constexpr (N0 < 32 && N >= 32) u = max(u, (uint32_t)__shfl_xor((int)u, 16));
-  if constexpr (N0 < 64 && N >= 64) u = max(u, (uint32_t)__shfl_xor((int)u, 32));
+// Unsigned maximum over groups of N lanes, up to a whole wave.
+template <int N>
+__device__ __forceinline__ float group_max_lanes(float x) {
+  uint32_t u = __float_as_uint(group_max<(N < 16 ? N : 16)>(x));
+  if constexpr (N >= 32) u = max(u, (uint32_t)__shfl_xor((int)u, 16));
+  if constexpr (N >= 64) u = max(u, (uint32_t)__shfl_xor((int)u, 32));
   return __uint_as_float(u);
 }
 
-template <int W, int DT, bool ANY>
+// The zero residual of rows r0 .. r0 + n - 1, by the lanes of a wave.
+__device__ __forceinline__ void zero_residual_rows(const RowsInit& p, int64_t r0, int64_t n, int lane) {
+  if (!p.resid) return;
+  const int64_t total = n * p.rk;
+  int8_t* z = p.resid + r0 * p.rk;
+  for (int64_t i = lane * 16; i < total; i += 1024) {
+    if (i + 16 <= total) {
+      st_stream16_u(z + i, u32x4{0u, 0u, 0u, 0u});
+    } else {
+      for (int64_t b = i; b < total; ++b) z[b] = 0;
+    }
+  }
+}
+
+// The zero residual scales, by `threads` threads of which this is number t.
+__device__ __forceinline__ void zero_scales(const RowsInit& p, int64_t t, int64_t threads) {
+  for (int64_t i = t; i < p.n_rscale; i += threads) p.rscale[i] = 0.0f;
+}
+
+// The EPL elements of type DT in N dwords, as fp32.
+template <int DT, int N, int EPL>
+__device__ __forceinline__ void decode_elements(const uint32_t (&w)[N], float (&v)[EPL]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if constexpr (DT == kF32) {
+      v[j] = __uint_as_float(w[j]);
+    } else {
+      v[2 * j] = act_decode<DT>(w[j] & 0xffffu);
+      v[2 * j + 1] = act_decode<DT>(w[j] >> 16);
+    }
+  }
+}
+
+// K = 16 * LPR, 16-byte aligned: 16 elements of a row per lane, its own bytes.
+// The arguments that every wave needs before its first load are the first twelve
+// dwords, which the dispatch preloads (with the number of waves read from the
+// implicit arguments instead, fp32 8 slots 5.06 against 4.72 us).
+template <int LPR, int DT, bool INIT>
+__global__ __launch_bounds__(256) void quantize_rows16_kernel(const char* __restrict__ x, int64_t stride_row_bytes,
+                                                              int64_t rows, int8_t* __restrict__ codes,
+                                                              float* __restrict__ scale, float qmax, uint32_t nwaves,
+                                                              const RowsInit init) {
+  constexpr int NP = DT == kF32 ? 4 : 2;  // 16-byte pieces of a lane's elements
+  constexpr int RPW = 64 / LPR;           // rows per wave
+  constexpr int K = 16 * LPR;
+  const int lane = threadIdx.x & 63;
+  const int c = lane % LPR;
+  const int g = lane / LPR;
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  for (int64_t r0 = wave * RPW; r0 < rows; r0 += (int64_t)nwaves * RPW) {
+    const int64_t row = r0 + g;
+    const bool valid = row < rows;
+    const u32x4* xr = reinterpret_cast<const u32x4*>(x + (valid ? row : rows - 1) * stride_row_bytes) + c * NP;
+    uint32_t bits[4 * NP];
+#pragma unroll
+    for (int w = 0; w < NP; ++w) {
+      const u32x4 a = xr[w];
+      bits[4 * w] = a.x, bits[4 * w + 1] = a.y, bits[4 * w + 2] = a.z, bits[4 * w + 3] = a.w;
+    }
+    if constexpr (INIT) zero_residual_rows(init, r0, min((int64_t)RPW, rows - r0), lane);
+    float v[16];
+    decode_elements<DT>(bits, v);
+    float am = fabsf(v[0]);
+#pragma unroll
+    for (int j = 1; j < 16; ++j) am = fmaxf(am, fabsf(v[j]));
+    am = group_max<LPR>(am);
+    const float s = round16<DT>(fmaxf(am, round16<DT>(kEps)) / qmax);
+    uint32_t yb[16];
+    if (DT != kF16 || s > 0.0f) {
+      const float inv = recip_rn(s);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        if constexpr (DT == kF32) {
+          (void)quantize<kExact>(v[j], s, inv, yb[j]);
+        } else {
+          const float q = round16<DT>(exact_quotient(v[j], s, inv));
+          yb[j] = __float_as_uint(fminf(fmaxf(rintf(q), -qmax), qmax) + kMagic);
+        }
+      }
+    } else {
+      // RN16(1e-12) = 0 in fp16: the row's scale rounded to 0, so x / 0 is +-inf
+      // (clamped to +-qmax) for x != 0 and NaN for x = 0, which the reference's
+      // int8 conversion turns into 0
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        yb[j] = __float_as_uint((v[j] > 0.0f ? qmax : v[j] < 0.0f ? -qmax : 0.0f) + kMagic);
+    }
+    if (valid) {
+      st_stream16(codes + row * K + c * 16,
+                  u32x4{pack_low_bytes(yb[0], yb[1], yb[2], yb[3]), pack_low_bytes(yb[4], yb[5], yb[6], yb[7]),
+                        pack_low_bytes(yb[8], yb[9], yb[10], yb[11]), pack_low_bytes(yb[12], yb[13], yb[14], yb[15])});
+      if (c == 0) scale[row] = s;
+    }
+  }
+  if constexpr (INIT) zero_scales(init, wave * 64 + lane, (int64_t)nwaves * 64);
+}
+
+// Any K from one lane's elements to 64 lanes': EPL elements per lane, the last
+// lane taking the row's last EPL, some of them its neighbour's too (the same codes).
+template <int W, int DT>
 __global__ __launch_bounds__(256) void quantize_rows_tile_kernel(const RowsParams p) {
   constexpr int EPL = DT == kF32 ? 4 : 8;
   constexpr int ESZ = DT == kF32 ? 4 : 2;
   constexpr int RPI = 64 / W;           // rows per wave instruction
   constexpr int U = 4;
   constexpr int ROWS = RPI * U;         // rows per wave and iteration
-  const int K = ANY ? p.K : W * EPL;
+  const int K = p.K;
   const int lane = threadIdx.x & 63;
   const int c = lane % W;
   const int g = lane / W;
-  const int e0 = ANY ? min(c * EPL, K - EPL) : c * EPL;
+  const int e0 = min(c * EPL, K - EPL);
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t nwaves = (int64_t)gridDim.x * 4;
-  for (int64_t i = wave * 64 + lane; i < p.n_rscale; i += nwaves * 64) p.rscale[i] = 0.0f;
+  zero_scales(p.init, wave * 64 + lane, nwaves * 64);
   for (int64_t r0 = wave * ROWS; r0 < p.rows; r0 += nwaves * ROWS) {
     u32x4 raw[U];
 #pragma unroll
@@ -115,70 +214,31 @@ __global__ __launch_bounds__(256) void quantize_rows_tile_kernel(const RowsParam
       const int64_t row = min(r0 + u * RPI + g, p.rows - 1);
       raw[u] = *reinterpret_cast<const u32x4_u*>(p.x + row * p.stride_row_bytes + e0 * ESZ);
     }
-    if (p.resid) {
-      const int64_t total = min((int64_t)ROWS, p.rows - r0) * p.rk;
-      int8_t* z = p.resid + r0 * p.rk;
-      for (int64_t i = lane * 16; i < total; i += 1024) {
-        if (i + 16 <= total) {
-          st_stream16_u(z + i, u32x4{0u, 0u, 0u, 0u});
-        } else {
-          for (int64_t b = i; b < total; ++b) z[b] = 0;
-        }
-      }
-    }
-    constexpr int DW = EPL / 4;
-    uint32_t w[U][DW];  // codes of the U rows, where whole 16-byte pieces are stored
+    zero_residual_rows(p.init, r0, min((int64_t)ROWS, p.rows - r0), lane);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t row = r0 + u * RPI + g;
       float v[EPL];
+      const uint32_t bits[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
+      decode_elements<DT>(bits, v);
+      float am = 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (DT == kF32) {
-          v[j] = __uint_as_float(raw[u][j]);
-        } else {
-          v[2 * j] = act_decode<DT>(raw[u][j] & 0xffffu);
-          v[2 * j + 1] = act_decode<DT>(raw[u][j] >> 16);
-        }
-      }
-      float am = ANY ? 0.0f : fabsf(v[0]);
-#pragma unroll
-      for (int j = ANY ? 0 : 1; j < EPL; ++j) am = fmaxf(am, fabsf(v[j]));
-      am = ANY ? group_max_from<1, W>(am) : group_max_from<16 / EPL, W>(group_fmax<16 / EPL>(am));
-      const float s = DT == kF32 ? fmaxf(am, kEps) / p.qmax
-                                 : round16<DT>(fmaxf(am, round16<DT>(kEps)) / p.qmax);
+      for (int j = 0; j < EPL; ++j) am = fmaxf(am, fabsf(v[j]));
+      am = group_max_lanes<W>(am);
+      const float s = round16<DT>(fmaxf(am, round16<DT>(kEps)) / p.qmax);
+      const bool plain = s >= 0x1p-100f && s < 0x1p125f;
+      const float inv = recip_rn(s);
       uint32_t yb[EPL];
-      if constexpr (ANY || DT != kF32) {
-        const bool plain = s >= 0x1p-100f && s < 0x1p125f;
-        const float inv = recip_rn(s);
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-          float q = exact_quotient(v[j], s, inv);
-          if constexpr (ANY) {
-            if (!plain) q = v[j] / s;
-            q = round16<DT>(q);
-            yb[j] = __float_as_uint((q != q ? 0.0f : fminf(fmaxf(rintf(q), -p.qmax), p.qmax)) + kMagic);
-          } else if (s > 0.0f) {
-            q = round16<DT>(q);
-            yb[j] = __float_as_uint(fminf(fmaxf(rintf(q), -p.qmax), p.qmax) + kMagic);
-          } else {
-            // fp16 only (RN16(1e-12) = 0): the row's scale rounded to 0, so x / 0
-            // is +-inf (clamped to +-qmax) for x != 0 and NaN for x = 0, which
-            // the reference's int8 conversion turns into 0
-            yb[j] = __float_as_uint((v[j] > 0.0f ? p.qmax : v[j] < 0.0f ? -p.qmax : 0.0f) + kMagic);
-          }
-        }
-      } else {
-        const float inv = recip_rn(s);
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) (void)quantize<kExact>(v[j], s, inv, yb[j]);
+      for (int j = 0; j < EPL; ++j) {
+        float q = exact_quotient(v[j], s, inv);
+        if (!plain) q = v[j] / s;
+        q = round16<DT>(q);
+        yb[j] = __float_as_uint((q != q ? 0.0f : fminf(fmaxf(rintf(q), -p.qmax), p.qmax)) + kMagic);
       }
-      const uint32_t w0 = pack_low_bytes(yb[0], yb[1], yb[2], yb[3]);
-      if constexpr (!ANY) {
-        w[u][0] = w0;
-        if constexpr (EPL == 8) w[u][1] = pack_low_bytes(yb[4], yb[5], yb[6], yb[7]);
-      } else if (row < p.rows && c * EPL < K) {
+      if (row < p.rows && c * EPL < K) {
         int8_t* dst = p.codes + row * K + e0;
+        const uint32_t w0 = pack_low_bytes(yb[0], yb[1], yb[2], yb[3]);
         if constexpr (EPL == 8) {
           st_stream8_u(dst, u32x2{w0, pack_low_bytes(yb[4], yb[5], yb[6], yb[7])});
         } else {
@@ -187,56 +247,47 @@ __global__ __launch_bounds__(256) void quantize_rows_tile_kernel(const RowsParam
       }
       if (row < p.rows && c == 0) p.scale[row] = s;
     }
-    if constexpr (!ANY) {
-      const bool odd = lane & 1;
-      // lanes 2i and 2i + 1 swap: the even one gets both lanes' codes of row u,
-      // the odd one those of row u + 1, in the order of their columns
-#pragma unroll
-      for (int u = 0; u < U; u += 2) {
-#pragma unroll
-        for (int i = 0; i < DW; ++i) {
-          const uint32_t x = dpp_u<kDppQuadXor1>(odd ? w[u][i] : w[u + 1][i]);
-          if (odd) w[u][i] = x;
-          else w[u + 1][i] = x;
-        }
-        if constexpr (EPL == 8) {
-          const int64_t row = r0 + (u + odd) * RPI + g;
-          if (row < p.rows)
-            st_stream16(p.codes + row * K + (c & ~1) * 8, u32x4{w[u][0], w[u][1], w[u + 1][0], w[u + 1][1]});
-        }
-      }
-      if constexpr (EPL == 4) {
-        // the pairs of a quad likewise: lane j of it gets row j's 16 codes
-        const bool hi = lane & 2;
-        const uint32_t x0 = dpp_u<kDppQuadXor2>(hi ? w[0][0] : w[2][0]);
-        const uint32_t x1 = dpp_u<kDppQuadXor2>(hi ? w[1][0] : w[3][0]);
-        const int64_t row = r0 + (c & 3) * RPI + g;
-        if (row < p.rows)
-          st_stream16(p.codes + row * K + (c & ~3) * 4,
-                      hi ? u32x4{x0, x1, w[2][0], w[3][0]} : u32x4{w[0][0], w[1][0], x0, x1});
-      }
-    }
   }
 }
 
-template <int W, bool ANY>
-void launch_rows_w(const RowsParams& p, int dtype, hipStream_t s) {
-  const int64_t waves = (p.rows + 64 / W * 4 - 1) / (64 / W * 4);
-  const dim3 grid((unsigned)std::min<int64_t>((waves + 3) / 4, 256 * 16)), b(256);
-  if (dtype == kF32) hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kF32, ANY>), grid, b, 0, s, p);
-  else if (dtype == kBF16) hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kBF16, ANY>), grid, b, 0, s, p);
-  else hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kF16, ANY>), grid, b, 0, s, p);
+// Workgroups of four waves, each of which takes rows_per_wave rows at a time.
+dim3 rows_grid(int64_t rows, int rows_per_wave, int most) {
+  const int64_t waves = (rows + rows_per_wave - 1) / rows_per_wave;
+  return dim3((unsigned)std::min<int64_t>((waves + 3) / 4, most));
 }
 
-template <bool ANY>
-void launch_rows(const RowsParams& p, int dtype, hipStream_t s) {
+template <int W>
+void launch_rows_any_w(const RowsParams& p, int dtype, hipStream_t s) {
+  const dim3 grid = rows_grid(p.rows, 64 / W * 4, 256 * 16), b(256);
+  if (dtype == kF32) hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kF32>), grid, b, 0, s, p);
+  else if (dtype == kBF16) hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kBF16>), grid, b, 0, s, p);
+  else hipLaunchKernelGGL((quantize_rows_tile_kernel<W, kF16>), grid, b, 0, s, p);
+}
+
+void launch_rows_any(const RowsParams& p, int dtype, hipStream_t s) {
   const int lanes = (p.K + (dtype == kF32 ? 4 : 8) - 1) / (dtype == kF32 ? 4 : 8);
-  if (lanes <= 2) launch_rows_w<2, ANY>(p, dtype, s);
-  else if (lanes <= 4) launch_rows_w<4, ANY>(p, dtype, s);
-  else if (lanes <= 8) launch_rows_w<8, ANY>(p, dtype, s);
-  else if (lanes <= 16) launch_rows_w<16, ANY>(p, dtype, s);
-  else if (lanes <= 32) launch_rows_w<32, ANY>(p, dtype, s);
-  else launch_rows_w<64, ANY>(p, dtype, s);
+  if (lanes <= 2) launch_rows_any_w<2>(p, dtype, s);
+  else if (lanes <= 4) launch_rows_any_w<4>(p, dtype, s);
+  else if (lanes <= 8) launch_rows_any_w<8>(p, dtype, s);
+  else if (lanes <= 16) launch_rows_any_w<16>(p, dtype, s);
+  else if (lanes <= 32) launch_rows_any_w<32>(p, dtype, s);
+  else launch_rows_any_w<64>(p, dtype, s);
+}
+
+template <int LPR, bool INIT>
+void launch_rows16_init(const RowsParams& p, int dtype, hipStream_t s) {
+  auto fn = dtype == kF32    ? quantize_rows16_kernel<LPR, kF32, INIT>
+            : dtype == kBF16 ? quantize_rows16_kernel<LPR, kBF16, INIT>
+                             : quantize_rows16_kernel<LPR, kF16, INIT>;
+  const dim3 grid = rows_grid(p.rows, 64 / LPR, 256 * 32);
+  hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, p.x, p.stride_row_bytes, p.rows, p.codes, p.scale, p.qmax, grid.x * 4,
+                     p.init);
+}
+
+template <int LPR>
+void launch_rows16(const RowsParams& p, int dtype, hipStream_t s) {
+  if (p.init.resid || p.init.n_rscale) launch_rows16_init<LPR, true>(p, dtype, s);
+  else launch_rows16_init<LPR, false>(p, dtype, s);
 }
 
 // The zero residual and scales of the paths that do not write them themselves.
@@ -490,10 +541,16 @@ extern "C" int ck_quantize_rows_init(const void* x, int x_dtype, int64_t stride_
     const bool aligned = ((reinterpret_cast<uintptr_t>(x) | (uintptr_t)(stride_row * esz) |
                            reinterpret_cast<uintptr_t>(codes)) & 15) == 0;
     if (K >= epl && K <= 64 * epl) {
-      const RowsParams p{static_cast<const char*>(x), stride_row * esz, rows, K, qmax, codes, scale, resid,
-                         resid_row_bytes, rscale, n_rscale};
-      if (aligned && (K == 16 || K == 32 || K == 64 || K == 128 || K == 256)) launch_rows<false>(p, x_dtype, s);
-      else launch_rows<true>(p, x_dtype, s);
+      const RowsParams p{static_cast<const char*>(x), stride_row * esz, rows, K, qmax, codes, scale,
+                         RowsInit{resid, resid_row_bytes, rscale, n_rscale}};
+      switch (aligned ? K : 0) {
+        case 16: launch_rows16<1>(p, x_dtype, s); break;
+        case 32: launch_rows16<2>(p, x_dtype, s); break;
+        case 64: launch_rows16<4>(p, x_dtype, s); break;
+        case 128: launch_rows16<8>(p, x_dtype, s); break;
+        case 256: launch_rows16<16>(p, x_dtype, s); break;
+        default: launch_rows_any(p, x_dtype, s); break;
+      }
       return check_launch("ck_quantize_rows");
     }
   }

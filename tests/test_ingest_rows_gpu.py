@@ -11,6 +11,7 @@ import pytest
 import torch
 
 import oracle
+from carrykernel_amd import _native
 from carrykernel_amd.vllm_integration import quantized_packed_decode as qpd
 
 pytestmark = pytest.mark.gpu
@@ -42,6 +43,27 @@ def test_every_k(K, dtype, S=3, HV=2, V=7):
         np.testing.assert_array_equal(sc.cpu().numpy(), c_ref)
         np.testing.assert_array_equal(ss.cpu().numpy(), s_ref)
         assert not rc.any() and not rs.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("rows", [1, 5, 333])
+def test_codes_and_scales_only(rows, K, dtype):
+    """ck_quantize_rows on aligned rows of a power of two, strided and with zero
+    rows; nothing past its outputs is written."""
+    g = torch.Generator().manual_seed(rows + K)
+    x = torch.zeros(rows, K + 16, dtype=dtype)
+    x[:, :K] = (torch.randn(rows, K, generator=g) * 0.2).to(dtype)
+    x[rows // 2] = 0.0
+    c_ref, s_ref = oracle.quantize_rows_in_dtype(x[:, :K].float().numpy(), NAMES[dtype], 127.0)
+    xd, codes = x.cuda(), torch.full((rows * K + 64,), 77, dtype=torch.int8, device="cuda")
+    scale = torch.full((rows + 16,), -1.0, device="cuda")
+    st = _native.lib().ck_quantize_rows(xd.data_ptr(), _native.dtype_code(xd, "x"), K + 16, rows, K, 127.0,
+                                        codes.data_ptr(), scale.data_ptr(), _native.stream_handle(0))
+    _native.check(st, "ck_quantize_rows")
+    np.testing.assert_array_equal(codes[:rows * K].view(rows, K).cpu().numpy(), c_ref)
+    np.testing.assert_array_equal(scale[:rows].cpu().numpy(), s_ref)
+    assert (codes[rows * K:] == 77).all() and (scale[rows:] == -1.0).all()
 
 
 @pytest.mark.parametrize("K", [100, 300])
