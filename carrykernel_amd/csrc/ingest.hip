@@ -372,43 +372,51 @@ __global__ __launch_bounds__(256) void quantize_rows_f64_kernel(const double* __
 // 16 bytes per row), two torch passes for values that were dropped and two
 // fills.
 // IEEE: the form of ck_statequant.h that the shape takes (ingest_ieee).
-struct ColsParams {
-  const float* x;
-  int V;
-  qs::ColTiles tiles;
-  int K;  // rows that exist (the kernel's K template argument is the padded count)
-  float qmax;
-  int8_t* codes;
-  float* scale;
+// The arguments that a workgroup needs before its first load are the first twelve
+// dwords, which the dispatch preloads. MORE: something is asked for besides codes
+// and scales.
+struct ColsInit {
   float* deq;      // or null
   char* e;         // or null
   int e_bytes;     // 1, 2 or 4
   float* e_scale;  // or null
 };
 
-template <int K, int FORM, bool MK, bool IEEE>
+struct ColsParams {
+  const float* x;
+  int8_t* codes;
+  float* scale;
+  int V, K;
+  qs::ColTiles tiles;
+  float qmax;
+  ColsInit init;
+};
+
+template <int K, int FORM, bool MK, bool IEEE, bool MORE>
 __global__ __launch_bounds__((qs::kThreadsFor<K, qs::TileShape<FORM, K>::GROUPS>)) void quantize_cols_tile_kernel(
-    const ColsParams p) {
+    const float* __restrict__ x, int8_t* __restrict__ codes, float* __restrict__ scale, int V, int nvt, int width,
+    int groups, uint32_t inv_groups, float qmax, int k_rows, const ColsInit init) {
   constexpr int CPT = qs::TileShape<FORM, K>::CPT;
   constexpr int S = qs::kSlicesFor<K>;
   constexpr int R = K / S;  // rows per slice
   constexpr int NC = qs::TileShape<FORM, K>::NC;
   __shared__ float red[S][NC];
-  const qs::TilePlace pl = qs::tile_place<FORM, S>(p.tiles, p.V, blockIdx.x % p.tiles.nvt);
+  const int m = nvt == 1 ? blockIdx.x : blockIdx.x / nvt;
+  const qs::ColTiles tiles{nvt, width, groups, inv_groups, (qs::TileForm)FORM};
+  const qs::TilePlace pl = qs::tile_place<FORM, S>(tiles, V, blockIdx.x - m * nvt);
   const int ks = pl.ks;
   const int lc = pl.cg * CPT;
   const int c0 = pl.col;
-  const int64_t m = blockIdx.x / p.tiles.nvt;
   const bool colok = c0 >= 0;
   const int r0 = ks * R;
-  const int KA = MK ? p.K : K;
-  const int64_t base = m * KA * p.V + (int64_t)r0 * p.V + c0;
+  const int KA = MK ? k_rows : K;  // rows that exist
+  const int64_t base = (int64_t)m * KA * V + (int64_t)r0 * V + c0;
   float v[R][CPT];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
 #pragma unroll
     for (int j = 0; j < CPT; ++j) v[r][j] = 0.0f;
-    if (colok && (!MK || r0 + r < KA)) qs::ld_f32<CPT>(p.x + base + (int64_t)r * p.V, v[r]);
+    if (colok && (!MK || r0 + r < KA)) qs::ld_f32<CPT>(x + base + (int64_t)r * V, v[r]);
   }
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
@@ -422,7 +430,7 @@ __global__ __launch_bounds__((qs::kThreadsFor<K, qs::TileShape<FORM, K>::GROUPS>
   float s[CPT], inv[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    s[j] = fmaxf(qs::ingest_amax<IEEE, S, NC>(red, lc + j), kEps) / p.qmax;
+    s[j] = fmaxf(qs::ingest_amax<IEEE, S, NC>(red, lc + j), kEps) / qmax;
     inv[j] = recip_rn(s[j]);
   }
 #pragma unroll
@@ -432,38 +440,49 @@ __global__ __launch_bounds__((qs::kThreadsFor<K, qs::TileShape<FORM, K>::GROUPS>
     float d[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      yb[j] = qs::ingest_code<IEEE>(v[r][j], s[j], inv[j], p.qmax);
+      yb[j] = qs::ingest_code<IEEE>(v[r][j], s[j], inv[j], qmax);
       d[j] = code_i8(yb[j], 0) * s[j];
     }
-    const int64_t i = base + (int64_t)r * p.V;
-    qs::st_b8<CPT>(p.codes + i, qs::pack_codes<CPT>(yb));
-    if (p.deq) qs::st_f32<CPT>(p.deq + i, d);
-    if (p.e) {
-      const uint32_t zw[(CPT + 1) / 2] = {};
-      const float zf[CPT] = {};
-      if (p.e_bytes == 1) qs::st_b8<CPT>(p.e + i, 0u);
-      else if (p.e_bytes == 2) qs::st_b16<CPT>(reinterpret_cast<uint16_t*>(p.e) + i, zw);
-      else qs::st_f32<CPT>(reinterpret_cast<float*>(p.e) + i, zf);
+    const int64_t i = base + (int64_t)r * V;
+    qs::st_b8<CPT>(codes + i, qs::pack_codes<CPT>(yb));
+    if constexpr (MORE) {
+      if (init.deq) qs::st_f32<CPT>(init.deq + i, d);
+      if (init.e) {
+        const uint32_t zw[(CPT + 1) / 2] = {};
+        const float zf[CPT] = {};
+        if (init.e_bytes == 1) qs::st_b8<CPT>(init.e + i, 0u);
+        else if (init.e_bytes == 2) qs::st_b16<CPT>(reinterpret_cast<uint16_t*>(init.e) + i, zw);
+        else qs::st_f32<CPT>(reinterpret_cast<float*>(init.e) + i, zf);
+      }
     }
   }
   if (ks == 0) {
-    qs::st_f32<CPT>(p.scale + m * p.V + c0, s);
-    if (p.e_scale) {
+    qs::st_f32<CPT>(scale + (int64_t)m * V + c0, s);
+    if (MORE && init.e_scale) {
       const float zf[CPT] = {};
-      qs::st_f32<CPT>(p.e_scale + m * p.V + c0, zf);
+      qs::st_f32<CPT>(init.e_scale + (int64_t)m * V + c0, zf);
     }
   }
 }
 
+template <int KP, int FORM, bool MK, bool IEEE>
+void launch_cols_kp(const ColsParams& p, int64_t M, hipStream_t s) {
+  const ColsInit& in = p.init;
+  auto fn = in.deq || in.e || in.e_scale ? quantize_cols_tile_kernel<KP, FORM, MK, IEEE, true>
+                                         : quantize_cols_tile_kernel<KP, FORM, MK, IEEE, false>;
+  const qs::ColTiles& t = p.tiles;
+  hipLaunchKernelGGL(fn, dim3((unsigned)(M * t.nvt)), dim3((unsigned)qs::tile_threads(t, qs::kSlicesFor<KP>)), 0, s,
+                     p.x, p.codes, p.scale, p.V, t.nvt, t.width, t.groups, t.inv, p.qmax, p.K, in);
+}
+
 template <int FORM, bool MK, bool IEEE>
 void launch_cols(const ColsParams& p, int KP, int64_t M, hipStream_t s) {
-  const dim3 g((unsigned)(M * p.tiles.nvt)), b((unsigned)qs::tile_threads(p.tiles, KP <= 128 ? 8 : 16));
   switch (KP) {
-    case 16: hipLaunchKernelGGL((quantize_cols_tile_kernel<16, FORM, MK, IEEE>), g, b, 0, s, p); break;
-    case 32: hipLaunchKernelGGL((quantize_cols_tile_kernel<32, FORM, MK, IEEE>), g, b, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((quantize_cols_tile_kernel<64, FORM, MK, IEEE>), g, b, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((quantize_cols_tile_kernel<128, FORM, MK, IEEE>), g, b, 0, s, p); break;
-    default: hipLaunchKernelGGL((quantize_cols_tile_kernel<256, FORM, MK, IEEE>), g, b, 0, s, p); break;
+    case 16: launch_cols_kp<16, FORM, MK, IEEE>(p, M, s); break;
+    case 32: launch_cols_kp<32, FORM, MK, IEEE>(p, M, s); break;
+    case 64: launch_cols_kp<64, FORM, MK, IEEE>(p, M, s); break;
+    case 128: launch_cols_kp<128, FORM, MK, IEEE>(p, M, s); break;
+    default: launch_cols_kp<256, FORM, MK, IEEE>(p, M, s); break;
   }
 }
 
@@ -590,8 +609,9 @@ extern "C" int ck_quantize_cols_init(const float* x, int64_t M, int K, int V, fl
   if (K <= 256 && !(ieee && qs::few_columns(M, K, V))) {
     return launch_slices(M, tiles.nvt, qs::tile_threads(tiles, KP <= 128 ? 8 : 16), [&](int64_t m0, int64_t n) {
       const int64_t i = m0 * K * V, c = m0 * V;  // the slice's first matrix and column
-      const ColsParams p{x + i, V, tiles, K, qmax, codes + i, scale + c, deq ? deq + i : nullptr,
-                         e ? static_cast<char*>(e) + i * e_bytes : nullptr, e_bytes, e_scale ? e_scale + c : nullptr};
+      const ColsParams p{x + i, codes + i, scale + c, V, K, tiles, qmax,
+                         ColsInit{deq ? deq + i : nullptr, e ? static_cast<char*>(e) + i * e_bytes : nullptr, e_bytes,
+                                  e_scale ? e_scale + c : nullptr}};
       switch (tiles.form) {
         case qs::kTileFull: launch_cols_form<qs::kTileFull>(p, KP, n, ieee, s); break;
         case qs::kTileAny: launch_cols_form<qs::kTileAny>(p, KP, n, ieee, s); break;
