@@ -202,10 +202,10 @@ void bind(uintptr_t decode, uintptr_t decode_to, uintptr_t quant_step, uintptr_t
 
 // A contiguous tensor of this dtype and shape on dev.
 bool is(const at::Tensor& t, at::ScalarType dtype, at::Device dev, std::initializer_list<int64_t> shape) {
-  if (t.scalar_type() != dtype || t.device() != dev || t.sizes() != at::IntArrayRef(shape.begin(), shape.size()) ||
-      !t.is_contiguous())
+  if (t.layout() != at::kStrided || t.scalar_type() != dtype || t.device() != dev ||
+      t.sizes() != at::IntArrayRef(shape.begin(), shape.size()) || !t.is_contiguous())
     return false;
-  return t.layout() == at::kStrided && t.data_ptr() != nullptr;
+  return t.data_ptr() != nullptr;
 }
 
 // gdn_quant_step_fused of carrykernel_amd/statequant/kernel.py for arguments it
@@ -325,8 +325,9 @@ PYBIND11_MODULE(_ck_front, m) {
   m.attr("QUANT_FAST") = kQuantFast;
   m.def("bind", &bind,
         "set the addresses of ck_gdn_packed_decode, ck_gdn_packed_decode_to, ck_gdn_quant_step and ck_gdn_fp32_step");
-  m.def("quant_step", &quant_step);
-  m.def("fp32_step", &fp32_step);
+  // with torch's own translation of its errors (out of memory stays torch.OutOfMemoryError)
+  m.def("quant_step", torch::wrap_pybind_function(quant_step));
+  m.def("fp32_step", torch::wrap_pybind_function(fp32_step));
   m.def("packed_decode", &packed_decode);
   m.def("launch_args", &launch_args);
 }

@@ -204,3 +204,36 @@ def test_python_front_end_raises_after_a_declined_call(front):
         qpd.quantized_gated_delta_rule_packed_decode(**c)
     with pytest.raises(_native.HipUnavailable):
         qpd.quantized_gated_delta_rule_packed_decode(**_case())
+
+
+@pytest.mark.parametrize("step", ["quant", "fp32"])
+def test_errors_of_the_statequant_front_are_not_swallowed(step, monkeypatch):
+    """A failed allocation or launch in the C++ front reaches the caller and is
+    not repeated in Python; only an argument of another type is declined."""
+    from carrykernel_amd.statequant import kernel as sq
+
+    class Front:
+        error, calls = torch.OutOfMemoryError("no memory"), 0
+
+        def quant_step(self, *args):
+            self.calls += 1
+            raise self.error
+        fp32_step = quant_step
+
+    front = Front()
+    monkeypatch.setattr(_native, "_front", front)
+    monkeypatch.setattr(_native, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(sq, "_is_gpu_tensor", lambda t: True)
+    x = [torch.zeros(1, 1, 16), torch.zeros(1, 1, 16), torch.zeros(1, 1, 4), torch.zeros(1, 1), torch.zeros(1, 1)]
+
+    def run():
+        if step == "fp32":
+            return sq.gdn_step_fused_fp32(torch.zeros(1, 1, 16, 4), *x)
+        return sq.gdn_quant_step_fused(torch.zeros(1, 1, 16, 4, dtype=torch.int8), torch.zeros(1, 1, 4),
+                                       torch.zeros(1, 1, 16, 4), None, *x)
+    with pytest.raises(torch.OutOfMemoryError):
+        run()
+    assert front.calls == 1
+    front.error = TypeError("incompatible function arguments")
+    with pytest.raises(_native.HipUnavailable):   # the Python checks go on
+        run()

@@ -21,6 +21,17 @@ def _inputs(B, HV, K, V, fmt):
                    torch.rand(B, HV, device="cuda")]
 
 
+@pytest.fixture
+def limited_memory():
+    """limited_memory(n): from now on no more than n bytes of new GPU memory."""
+    def limit(n):
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + n) / total)
+    yield limit
+    torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 def _bits(ts):
     return [None if t is None else t.contiguous().view(torch.uint8).cpu() for t in ts]
 
@@ -61,3 +72,12 @@ def test_same_as_python(fmt, K, V, monkeypatch):
     _same(got32, sq.gdn_step_fused_fp32(h, *x))
     _same(got_b, sq.gdn_quant_step_fused(*state, *[t.float() for t in xb], res_fmt=fmt))
     _same(got_s, sq.gdn_quant_step_fused(*state, *x, res_fmt=fmt))
+
+
+def test_out_of_memory_is_torch_s(limited_memory):
+    """An output that cannot be allocated raises torch.OutOfMemoryError."""
+    state, x = _inputs(16, 16, 256, 256, sq.RES_FP32)
+    assert _native._front is not None
+    limited_memory(1 << 20)
+    with pytest.raises(torch.OutOfMemoryError):
+        sq.gdn_quant_step_fused(*state, *x)
