@@ -81,3 +81,19 @@ def test_out_of_memory_is_torch_s(limited_memory):
     limited_memory(1 << 20)
     with pytest.raises(torch.OutOfMemoryError):
         sq.gdn_quant_step_fused(*state, *x)
+
+
+def test_decode_without_room_for_the_converted_inputs(limited_memory):
+    """bf16 inputs whose fp32 copies for all tokens do not fit run token by
+    token, to the same bits (the copies take 136 MB, the outputs 2 MB)."""
+    T, B, HV, K, V = 512, 8, 32, 128, 4
+    g = torch.Generator(device="cuda").manual_seed(2)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    h0 = r(B, HV, K, V) * 0.1
+    x = [t.to(torch.bfloat16) for t in (r(T, B, HV, K) * 0.1, r(T, B, HV, K) * 0.1, r(T, B, HV, V),
+                                        torch.rand(T, B, HV, device="cuda"), torch.rand(T, B, HV, device="cuda"))]
+    ref = [None if t is None else t.cpu() for t in sq.gdn_quant_decode_fused(h0, *x, T)]
+    limited_memory(64 << 20)
+    assert sq._decode_one_launch(h0, tuple(x), T, 8, sq.RES_FP32, "fast") is None
+    got = sq.gdn_quant_decode_fused(h0, *x, T)
+    _same(tuple(got), tuple(ref))
