@@ -223,13 +223,16 @@ def test_errors_of_the_statequant_front_are_not_swallowed(step, monkeypatch):
     front = Front()
     monkeypatch.setattr(_native, "_front", front)
     monkeypatch.setattr(_native, "stream_handle", lambda device: 0)
-    monkeypatch.setattr(sq, "_is_gpu_tensor", lambda t: True)
+
+    class Gpu(torch.Tensor):
+        is_cuda = True
+
     x = [torch.zeros(1, 1, 16), torch.zeros(1, 1, 16), torch.zeros(1, 1, 4), torch.zeros(1, 1), torch.zeros(1, 1)]
 
     def run():
         if step == "fp32":
-            return sq.gdn_step_fused_fp32(torch.zeros(1, 1, 16, 4), *x)
-        return sq.gdn_quant_step_fused(torch.zeros(1, 1, 16, 4, dtype=torch.int8), torch.zeros(1, 1, 4),
+            return sq.gdn_step_fused_fp32(torch.zeros(1, 1, 16, 4).as_subclass(Gpu), *x)
+        return sq.gdn_quant_step_fused(torch.zeros(1, 1, 16, 4, dtype=torch.int8).as_subclass(Gpu), torch.zeros(1, 1, 4),
                                        torch.zeros(1, 1, 16, 4), None, *x)
     with pytest.raises(torch.OutOfMemoryError):
         run()
