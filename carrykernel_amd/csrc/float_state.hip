@@ -18,9 +18,11 @@
 // own bytes touched every line of the wave's rows in every instruction. HBM is
 // the bound (the swaps are 2 VALU operations per fp32 element each way).
 // Against the persistent kernel with a register prefetch and each lane's own
-// bytes (HV=32, V=128, us): bf16 K=128 B=64 31.7 -> 22.9, B=128 60.7 -> 55.4 (4.9
-// TB/s), K=256 B=48 45.7 -> 40.2; fp32 K=128 B=8 12.6 -> 7.4, B=64 65.1 -> 50.5,
-// B=128 122.6 -> 98.3 (5.6 TB/s), K=256 B=48 91.9 -> 72.4.
+// bytes (HV=32, V=128, us), state sets that a last-level cache of 256 MB holds in
+// part: bf16 K=128 B=64 31.7 -> 22.9 (192 MB in turn; with cold sets 30.3 -> 30.3, no
+// gain); larger ones: bf16 B=128 60.7 -> 55.4 (4.9 TB/s), K=256 B=48 45.7 -> 40.2;
+// fp32 K=128 B=8 12.6 -> 7.4, B=64 65.1 -> 50.5, B=128 122.6 -> 98.3 (5.6 TB/s), K=256
+// B=48 91.9 -> 72.4.
 #include <hip/hip_runtime.h>
 
 #include "ck_capi_common.h"

@@ -57,8 +57,9 @@ __device__ __forceinline__ float round16_rt(int dt, float x) {
 //    of any alignment, four rows in flight: IEEE quotients and the clamp (infinities,
 //    scales that are no normal number), NaN codes 0 and NaNs no part of the amax.
 // 16-bit dtypes in their own precision: RN16 after every fp32 operation.
-// HBM bounds large fp32 states (5.6 TB/s at 257 slots of [32, 128, 128]), HBM and
-// about 12 VALU operations an element 16-bit ones (6.6 TB/s). Row-level work is done
+// HBM bounds large fp32 states (5.6 TB/s at 257 slots of [32, 128, 128]); the VALU,
+// with 16 operations an element (0.25 instructions per SIMD and cycle, fp32 0.06),
+// 16-bit ones (6.7 TB/s). Row-level work is done
 // once per 16 elements: 4 or 8 elements per lane in one access each, with the codes
 // exchanged into 16-byte stores, were slower (us, so / now: 257 slots bf16 70.2 /
 // 60.6, fp16 67.4 / 60.3, fp32 123.0 / 121.0; 8 slots bf16 6.0 / 4.2), and so were

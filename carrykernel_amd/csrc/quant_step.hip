@@ -24,8 +24,8 @@
 // amax, and store nothing), so the sums keep the KP slice order.
 //
 // Columns per thread: four, one vector access per row at any alignment, with as
-// many column groups in a workgroup as the tile's width needs (ck_statequant.h,
-// TileForm); one column for V < 4 only. Before, any V but a multiple of 4 with
+// many column groups in a workgroup as the tile's width needs or 32 (ck_tiles.h,
+// TileForm); one column for V < 4 and from 2^32 elements on. Before, any V but a multiple of 4 with
 // 16-byte aligned tensors took one column per thread, 32 to a workgroup (HV=32, us
 // a call: K=100 V=130 B=16 fp32 residual 28.0 -> 18.2, fp16 25.1 -> 15.8, where the
 // host's share is 15; K=256 V=130 B=16 fp32 70.0 -> 51.3, int8 48.5 -> 39.4;

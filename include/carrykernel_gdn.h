@@ -248,9 +248,11 @@ int ck_gdn_packed_decode_float_state(const void* mixed_qkv, int qkv_dtype, int64
  * In-place use (h_out == h_in, e_out == e_in, ...) is allowed.
  * Requirements: K in 1..256 (rows past K zero-padded to max(16, next_pow2(K)),
  *   whose K-slices fix the reduction order); any V >= 1; fp32 tensors 4-byte
- * and the residual element-size aligned. V % 4 == 0 with 16-byte aligned
- * tensors takes one vector access per 4 columns, anything else one access
- * per column (statequant/kernel.py:277-279 masks offs_v < V the same way).
+ * and the residual element-size aligned. A row's columns are accessed four
+ * at a time at that alignment, the last four of a V that is no multiple of 4
+ * sharing columns with their neighbours in the same workgroup; one by one for
+ * V < 4 and for matrices of 2^32 elements or more (statequant/kernel.py:277-279
+ * masks offs_v < V).
  */
 int ck_gdn_quant_step(const int8_t* h_in, const float* scale_in, const void* e_in,
                       const float* e_scale_in,
