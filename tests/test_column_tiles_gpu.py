@@ -1,4 +1,4 @@
-"""The statequant step's column tiles (ck_statequant.h, TileForm): V below one
+"""The statequant step's column tiles (ck_tiles.h, TileForm): V below one
 4-column group, around one group, one wave, the widest tile and two tiles, where
 the last thread shares columns with its neighbour, in place and out of place, on
 tensors one element off alignment. Bit for bit against the oracle."""
